@@ -12,15 +12,15 @@
 // One workgroup of 512 threads (8 wave64) walks the chunks of one (sequence, head) and keeps everything of a chunk
 // on chip: the only HBM traffic is q, k, v, g, beta in, o out, and the state in / out / checkpoints.  The next
 // chunk's inputs are prefetched into registers while the current chunk is processed.  Per chunk:
-//   P0  raw rows -> LDS (gate), row norms (DPP)          thread (r = tid / 8, channels 16 (tid % 8) .. + 15)
-//   P1  in-chunk gate cumsum, 4 segments of 16 rows      thread (channel tid % 128, segment tid / 128)
-//   P2  per-element factors fi = e^{Gamma_i - Gamma_m}, fj = 1 / fi with m the middle row of the 16-row block,
-//       and the per-channel block factors (a, b, x, y, decay) -- two exponentials per element
+//   P0-P2  the wave's 8 rows (lane: 4 rows x 4 channels) to gated operands in registers: gate activation, running
+//       gate sums, row norms, per-element factors fi = e^{Gamma_i - Gamma_m}, fj = 1 / fi with m the middle row of the
+//       16-row block (two exponentials per element), all before the chunk's first barrier; then k^ fi, k^ fj and q^ fi
+//       go to LDS and the per-channel block factors (a, b, x, y, decay) are formed from the waves' gate totals
 //   P4  Gram tiles on MFMA: the four diagonal 16 x 16 blocks from bf16 hi + lo operands (3 MFMAs: hi.hi + hi.lo +
 //       lo.hi; their gated operands span e^{+-8|g|}), the six off-diagonal blocks from fp16 operands <= 1 (the
 //       reference point is the last row before the row block); each diagonal wave then inverts its block,
 //       (I + L_II)^-1 by forward substitution in fp32, while the off-diagonal waves finish
-//   P5  Q e^Gamma, K e^{Gamma_c - Gamma} and beta V to LDS in the walk's operand layouts
+//   P5  Q e^Gamma and K e^{Gamma_c - Gamma} (from the lane's registers) to LDS in the walk's operand layouts
 //   P6  W and U by block forward substitution on MFMA: X_I = T_II (B_I - sum_{J<I} A_IJ X_J); wave w owns key
 //       channels [16w, 16w+16) of W and value columns [16w, 16w+16) of U, so no wave waits for another
 //   P7  the walk: wave w keeps the 128 x 16 slice S[:, 16w:16w+16] in fp32 registers (MFMA C layout) for the whole
@@ -44,29 +44,46 @@ namespace {
 
 constexpr int PF_THREADS = 512;
 
-// LDS layout (bytes).  Region A: gate / Gamma fp32 [64][132], then k^ fi fp32 [64][132].  Region B: q^ fi fp32
-// [64][132], then Q~ fp16 [64][136] and W fp16 [64][136].  Region C: k^ fj fp32 [64][132], then Kd^T fp16
-// [128][72].  The row paddings keep the scattered two-byte stores of the layouts and the column reads free of bank
-// conflicts and every MFMA fragment at a constant offset from its lane's base.  On gfx950 the 16-byte fragment reads
-// of these rows still take two LDS passes (SQ_LDS_BANK_CONFLICT); swizzled rows that read in one pass measured no
-// faster, since the kernel's phases wait on VALU issue, not on the LDS.
+// LDS layout (bytes).  Region A: k^ fi fp32 [64][132].  Region B: q^ fi fp32 [64][132], then Q~ fp16 [64][144] and W
+// fp16 (two half arrays [64][72]).  Region C: k^ fj fp32 [64][132], then Kd^T fp16 (two half arrays [128][40]).
+//
+// Bank conflicts.  A 16-byte LDS read of gfx950 serves 16 lanes a cycle (256 B per clock and CU when free of conflicts):
+// of lanes 16 g + m, those with m in {0-3, 12-15} of one g and those with m in {4-11} of the g beside it (g ^ 1).  A
+// fragment read (row m, 16-byte slot of the lane's g) is free of conflicts when those 16 (row, slot) pairs fall on the
+// 16 distinct slots of the 64 banks; plain padded rows (272, 528, 144 bytes) put two pairs on some slot and take twice
+// the cycles (8.4 against 4.2 per wave instruction).  So:
+//   - fp32 rows of 528 bytes: the lanes of g and g ^ 1 read channels 64 apart (gram_c0; any bijection of a step's K
+//     indices serves, as all operands of a product use the same one);
+//   - Q~ rows of 288 bytes (two slots of shift a row: the even g on even slots, the odd g on odd ones);
+//   - W, A_qk and Kd^T as two half arrays, the slots of the even g and of the odd g, with rows of an odd number of
+//     slots, a multiple of 256 bytes apart (their 8-byte writes, 16 consecutive lanes at a time, stay free of
+//     conflicts too, which 288- and 160-byte rows would double).
+// Measured with an LDS probe; the chunk's LDS time falls from 11.2 k to 8.4 k cycles of the CU by these figures (config 1 0.747 ->
+// 0.700 ms).
 constexpr int RS32 = 132;   // fp32 rows of 128
+constexpr int RSQ = 144;    // Q~ rows (fp16)
+constexpr int RSW = 72;     // rows of a half array of W (fp16, 64 channels)
+constexpr int RST = 40;     // rows of a half array of A_qk or Kd^T (fp16, 32 tokens)
 constexpr int RS16 = 136;   // fp16 rows of 128
 constexpr int RS16S = 72;   // fp16 rows of 64
+constexpr int RSF = 132;    // factor rows: channel c at c + 4 (c / 64) (see f_at)
+constexpr int W_HALF = 64 * RSW, AQ_HALF = 64 * RST, KD_HALF = 128 * RST;  // elements of a half array
 constexpr int LDS_A = 0;
 constexpr int LDS_B = 33792;
-constexpr int LDS_BV = LDS_B + 17408;
-constexpr int LDS_C = 68608;
-constexpr int LDS_W = 102400;
-constexpr int LDS_AQ = 119808;
-constexpr int LDS_AK = 129024;
-constexpr int LDS_GM = 138240;      // the gate cumsum's block middle rows 16 I + 7 [4][128] fp32 (2 KiB; 2304 bytes free)
-constexpr int LDS_F = 142592;
-constexpr int LDS_WT = 151808;
-constexpr int LDS_BETA = 153856;
-constexpr int LDS_DT = 154112;    // dt_bias of the head (gate-in-kernel) fp32 [128]
-constexpr int LDS_L = 154624;     // A_kk diagonal blocks, transposed: [block][column][row], rows padded to 20
-constexpr int LDS_TOTAL = 159744;
+constexpr int LDS_BV = LDS_B + 64 * RSQ * 2;
+constexpr int LDS_C = LDS_BV + 2 * W_HALF * 2;
+constexpr int LDS_VT = LDS_C + 33792;           // V^T bf16 [128][72] (channel rows in ch_row order)
+constexpr int LDS_AQ = LDS_VT + 128 * RS16S * 2;
+constexpr int LDS_AK = LDS_AQ + 2 * AQ_HALF * 2;
+constexpr int LDS_F = LDS_AK + 64 * RS16S * 2;
+constexpr int LDS_WT = LDS_F + 18 * RSF * 4;    // gate totals of the 8 waves' rows [8][128]; PREC: then T_II's low parts
+constexpr int LDS_BETA = LDS_WT + 8 * 128 * 4;
+constexpr int LDS_DT = LDS_BETA + 64 * 4;       // An dt_bias of the head (gate-in-kernel) fp32 [128]
+constexpr int LDS_L = LDS_DT + 128 * 4;         // A_kk diagonal blocks, transposed: [block][column][row], rows padded to 20
+constexpr int LDS_TOTAL = LDS_L + 4 * 16 * 20 * 4;
+static_assert(LDS_TOTAL <= 160 * 1024, "one workgroup per CU");
+static_assert(W_HALF * 2 % 256 == 0 && AQ_HALF * 2 % 256 == 0 && KD_HALF * 2 % 256 == 0, "half arrays share their banks");
+static_assert(2 * KD_HALF * 2 <= 33792, "Kd^T fits region C");
 // per-channel factor rows of LDS_F
 constexpr int F_A = 0;      // a_I = e^{Gamma_m(I) - Gamma_{16I-1}}, I = 1..3          (rows 0..2)
 constexpr int F_B = 3;      // b_IJ = e^{Gamma_{16I-1} - Gamma_m(J)}, row 3 + I(I-1)/2 + J (rows 3..8)
@@ -111,6 +128,17 @@ __device__ __forceinline__ f32x4 mfma16(f16x4 a, f16x4 b, f32x4 c) {
 // storage position of index q (0..31) inside a permuted 32-block: q = 16h + 4g + e  ->  8g + 4h + e
 __device__ __forceinline__ int pos32(int q) { return ((q >> 2) & 3) * 8 + ((q >> 4) << 2) + (q & 3); }
 __device__ __forceinline__ int pos64(int q) { return (q & 32) + pos32(q & 31); }
+// element offset of stored position p (= 32 s + 8 g + i) of a row in two half arrays of `half` elements with rows of
+// `stride`: the slots of even g in the first, of odd g in the second
+__device__ __forceinline__ int half_at(int row, int p, int stride, int half) {
+    const int g = (p >> 3) & 3;
+    return (g & 1) * half + row * stride + 16 * (p >> 5) + 8 * (g >> 1) + (p & 7);
+}
+// first channel of lane group g in K step s of the Gram products
+__device__ __forceinline__ int gram_c0(int s, int g) { return 64 * (g & 1) + 32 * (g >> 1) + 8 * s; }
+// channel c in a factor row: the two 64-channel halves sit 4 floats apart in the banks, so that the lane groups of
+// gram_c0 read distinct slots
+__device__ __forceinline__ int f_at(int c) { return c + 4 * (c >> 6); }
 // Channel swizzle of the fp32 row arrays (gate / Gamma, q^ fi, k^ fi, k^ fj; 132-float rows): logical channel c is
 // stored at c ^ (((c >> 5) & 3) << 2), i.e. the four 16-byte slots of the 16-channel segment of raw thread cb are
 // permuted by slot ^= cb >> 1.  The eight raw threads of a row then write 16-byte slots on distinct banks (unswizzled,
@@ -135,12 +163,12 @@ __device__ __forceinline__ float sigmoid_rcp(float x) { return __builtin_amdgcn_
 // 8 tokens, inside 2^{+-104} for g >= -9, where the factors and the low halves of their bf16 pairs stay normal (the
 // MFMAs flush subnormal operands; at -11 the factors reach 2^-127).  The state change this makes is below e^{-9} =
 // 1.2e-4 of the affected channel's value (a decay of e^{-9} instead of a smaller one).  NaN passes through unchanged.
-__device__ __forceinline__ float clamp_decay(float g) { return g < KDA355_MIN_LOG_DECAY ? KDA355_MIN_LOG_DECAY : g; }
+__device__ __forceinline__ float clamp_decay(float g) { return __builtin_elementwise_maximum(g, KDA355_MIN_LOG_DECAY); }
 // the same limit for a log-decay already in log2 units
 constexpr float LOG2E = 1.4426950408889634f;
 __device__ __forceinline__ float clamp_decay2(float g) {
     constexpr float lim = KDA355_MIN_LOG_DECAY * LOG2E;
-    return g < lim ? lim : g;
+    return __builtin_elementwise_maximum(g, lim);
 }
 // Gate-in-kernel constant of a head: An = -e^{A_log} log2(e), so that e^{-e^{A_log} (x + dt_bias)} =
 // 2^{An x + An dt_bias} is one FMA (An dt_bias per channel sits in LDS) and one v_exp_f32
@@ -264,6 +292,193 @@ __device__ __forceinline__ void unpack16(const u32x4 (&w)[2], float (&f)[16]) {
         }
 }
 
+// Raw inputs of one chunk for one lane.  Wave w owns the chunk's rows 8 w .. 8 w + 7; lane l of it the rows
+// row0 + j (row0 = 8 w + 4 (l / 32), j = 0 .. 3) at channels 4 (l % 32) .. + 3.
+struct RawRows {
+    u32x2 q[4], k[4], v[4];
+    u32x4 g[4];     // fp32 log-decay, or the bf16 raw gate of the 4 channels in the first two words
+    uint32_t beta;  // row 8 w + l % 8: fp32 bits, or the bf16 raw beta in the low half (converted when consumed)
+};
+
+__device__ __forceinline__ u32x2 bload8(__amdgpu_buffer_rsrc_t rs, int off) {
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+}
+
+// One chunk's rows for this lane (row0, c4 = l % 32); rows >= L read as zeros.  The next chunk's rows are issued in
+// three parts in three phases (q and k; v and beta; the gate): the 80 KiB a chunk loads take ~1.3 k cycles of the CU's
+// address unit, and issued at once they stall the waves that issue them.
+__device__ __forceinline__ void load_rows_qk(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows& x) {
+    const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
+    const int64_t qp = p.qkv_rs * 2;
+    const int qo = row0 * (int)qp + 8 * c4;
+    const __amdgpu_buffer_rsrc_t rq = rows_rsrc(p.q + o, L, qp, 256);
+    const __amdgpu_buffer_rsrc_t rk = rows_rsrc(p.k + o, L, qp, 256);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x.q[j] = bload8(rq, qo + j * (int)qp);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x.k[j] = bload8(rk, qo + j * (int)qp);
+}
+__device__ __forceinline__ void load_rows_vb(const PfParams& p, int h, int t0, int L, int row0, int c4, bool RB,
+                                             RawRows& x) {
+    const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
+    const int64_t qp = p.qkv_rs * 2;
+    const int qo = row0 * (int)qp + 8 * c4;
+    const __amdgpu_buffer_rsrc_t rv = rows_rsrc(p.v + o, L, qp, 256);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x.v[j] = bload8(rv, qo + j * (int)qp);
+    const int es = RB ? 2 : 4;
+    const int64_t bp = p.beta_rs * es;
+    const int bo = ((row0 & ~7) + (c4 & 7)) * (int)bp;
+    const __amdgpu_buffer_rsrc_t rb =
+        rows_rsrc(reinterpret_cast<const unsigned char*>(p.beta) + ((int64_t)t0 * p.beta_rs + h) * es, L, bp, es);
+    x.beta = RB ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rb, bo, 0, 0)
+                : __builtin_amdgcn_raw_buffer_load_b32(rb, bo, 0, 0);
+}
+template <bool RG>
+__device__ __forceinline__ void load_rows_g(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows& x) {
+    const int64_t go = (int64_t)t0 * p.g_rs + (int64_t)h * D;
+    if (RG) {
+        const int64_t gp = p.g_rs * 2;
+        const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const uint16_t*>(p.g) + go, L, gp, 256);
+        const int off = row0 * (int)gp + 8 * c4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u32x2 y = bload8(rg, off + j * (int)gp);
+            x.g[j] = u32x4{y.x, y.y, 0u, 0u};
+        }
+    } else {
+        const int64_t gp = p.g_rs * 4;
+        const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const float*>(p.g) + go, L, gp, 512);
+        const int off = row0 * (int)gp + 16 * c4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x.g[j] = bload16(rg, off + j * (int)gp);
+    }
+}
+template <bool RG>
+__device__ __forceinline__ void load_rows(const PfParams& p, int h, int t0, int L, int row0, int c4, bool RB, RawRows& x) {
+    load_rows_qk(p, h, t0, L, row0, c4, x);
+    load_rows_vb(p, h, t0, L, row0, c4, RB, x);
+    load_rows_g<RG>(p, h, t0, L, row0, c4, x);
+}
+
+// Row of channel k in the channel-major arrays (V^T, Kd^T): the lanes' 8-byte writes (channels 4 c4 + e of 32 lanes)
+// then fall on twice the banks that plain rows would give them, and a 16-channel tile still reads distinct banks.
+__device__ __forceinline__ int ch_row(int k) { return 16 * (k >> 4) + ((k & 15) ^ (k >> 4)); }
+
+// 1 / max(|x|, 1e-6) (F.normalize, kda/mi350x/reference.py:59-60) of the lane's 4 q and 4 k rows, each row held by the
+// 32 lanes of a half wave.  Sums of squares straight from the packed bf16 pairs (v_dot2c_f32_bf16: the products are
+// exact in fp32); the halving exchange over the two 16-lane rows leaves 4 values to reduce by DPP instead of 8.
+// rsqrt(max(|x|^2, 1e-12)) through v_rsq_f32 (the IEEE sqrt is a sequence).
+__device__ __forceinline__ void row_norms(const RawRows& x, float (&rq)[4], float (&rk)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float sq = 0.f, sk = 0.f;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            // element copies first: a bit cast of the vector element itself loses its index in this compiler
+            const uint32_t wq = x.q[j][i], wk = x.k[j][i];
+            const bf16x2_t qp = __builtin_bit_cast(bf16x2_t, wq), kp = __builtin_bit_cast(bf16x2_t, wk);
+            sq = __builtin_amdgcn_fdot2_f32_bf16(qp, qp, sq, false);
+            sk = __builtin_amdgcn_fdot2_f32_bf16(kp, kp, sk, false);
+        }
+        // even 16-lane rows continue with q's sum, odd ones with k's
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(sq), __float_as_uint(sk), false, false);
+        const float s = sum16(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+        const uint32_t n = __float_as_uint(__builtin_amdgcn_rsqf(fmaxf(s, 1e-12f)));
+        const auto b = __builtin_amdgcn_permlane16_swap(n, n, false, false);
+        rq[j] = __uint_as_float(b[0]);
+        rk[j] = __uint_as_float(b[1]);
+    }
+}
+
+// A chunk's rows from the prefetched registers to the gated operands, before any barrier: everything here needs only
+// the wave's own 8 rows.  The reference row of a 16-row block is its row 7, the last row of the block's even wave, so
+// Gamma_r - Gamma_m is the lane's running sum of g (odd wave), or that sum minus the wave's total (even wave); only the
+// block factors need the other waves' totals (sWt, read behind the next barrier).  Writes V^T, beta and the wave's
+// gate totals to LDS; returns k^ fi, k^ fj and q^ fi of the lane's 4 rows (fi = e^{Gamma_r - Gamma_m}, fj = 1 / fi).
+// Bound by the SIMD's VALU (two waves per SIMD, half of these instructions at half or quarter rate).  The form before
+// summed the gate in channel threads through LDS: one more barrier, 64 KiB more LDS traffic a chunk, 16-channel lanes
+// whose Kd^T and v accesses were two bytes wide.  Measured: 96 heads x 8,192 tokens 591 -> 566 us, 38,881 tokens x 32
+// heads 761 -> 747 us.
+template <bool RG>
+__device__ __forceinline__ void chunk_front(const RawRows& x, int w, int lane, int L, bool RB, bool NORM, float An,
+                                            float lb, const float* sDT, float* sWt, float* sBeta, uint16_t* sVt,
+                                            int vt_stride, f32x4 (&kfi)[4], f32x4 (&kfj)[4], f32x4 (&qfi)[4]) {
+    const int c4 = lane & 31, hf = lane >> 5, row0 = 8 * w + 4 * hf;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {  // V^T: 4 rows of one channel per write
+        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+        const uint32_t v0 = x.v[0][e >> 1], v1 = x.v[1][e >> 1], v2 = x.v[2][e >> 1], v3 = x.v[3][e >> 1];
+        *reinterpret_cast<u32x2*>(&sVt[ch_row(4 * c4 + e) * vt_stride + row0]) =
+            u32x2{__builtin_amdgcn_perm(v1, v0, sel), __builtin_amdgcn_perm(v3, v2, sel)};
+    }
+    {
+        const int br = 8 * w + (lane & 7);
+        const float bx = RB ? sigmoid_rcp(bf2f(x.beta)) : __uint_as_float(x.beta);
+        if (lane < 8) sBeta[br] = (br >= L) ? 0.f : bx;
+    }
+    float d[4][4];  // [row][channel]: the clamped log-decay, then Gamma_r - Gamma_m in log2 units
+    if (RG) {
+        // g log2(e) = lb log2(e) sigmoid(e^{A_log} (x + dt_bias)), the sigmoid as 1 / (1 + 2^{An x + An dt}) (one FMA,
+        // v_exp_f32, one add, v_rcp_f32), already in log2 units.  Every row is computed; rows >= L get a zero
+        // multiplier (their raw gate reads as 0, so the sigmoid is finite).
+        const f32x4 adt = *reinterpret_cast<const f32x4*>(&sDT[4 * c4]);  // An dt_bias
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float lbm = (row0 + j < L) ? lb * LOG2E : 0.f;
+            const uint32_t w0 = x.g[j][0], w1 = x.g[j][1];
+            const float rg[4] = {bf2f(w0 & 0xffffu), bf2f(w0 >> 16), bf2f(w1 & 0xffffu), bf2f(w1 >> 16)};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                d[j][e] = clamp_decay2(lbm * __builtin_amdgcn_rcpf(1.0f + exp2_(fmaf(An, rg[e], adt[e]))));
+        }
+    } else {  // natural-log units; the running sums scale by log2(e) as they add
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t gw = x.g[j][e];
+                d[j][e] = clamp_decay(__uint_as_float(gw));
+            }
+    }
+    // the lane's sum starts behind the rows of its wave that precede it (odd wave), or at minus its own and the later
+    // rows' sum (even wave): s1 lo + s2 hi, with lo / hi the sums of the wave's first and last 4 rows
+    const bool odd = (w & 1) != 0;
+    const float unit = RG ? 1.f : LOG2E;
+    const float s1 = (odd ? (hf ? 1.f : 0.f) : (hf ? 0.f : -1.f)) * unit, s2 = odd ? 0.f : -unit;
+    f32x4 tot;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t t = __float_as_uint((d[0][e] + d[1][e]) + (d[2][e] + d[3][e]));
+        const auto r = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+        const float lo = __uint_as_float(r[0]), hi = __uint_as_float(r[1]);
+        tot[e] = RG ? lo + hi : (lo + hi) * LOG2E;
+        float a = fmaf(s1, lo, s2 * hi);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[j][e] = a = RG ? a + d[j][e] : fmaf(d[j][e], LOG2E, a);
+    }
+    *reinterpret_cast<f32x4*>(&sWt[w * 128 + 4 * c4]) = tot;  // both half waves hold it
+    float rq[4], rk[4];
+    if (NORM) row_norms(x, rq, rk);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t q0 = x.q[j][0], q1 = x.q[j][1], k0 = x.k[j][0], k1 = x.k[j][1];
+        float qf[4] = {bf2f(q0 & 0xffffu), bf2f(q0 >> 16), bf2f(q1 & 0xffffu), bf2f(q1 >> 16)};
+        float kf[4] = {bf2f(k0 & 0xffffu), bf2f(k0 >> 16), bf2f(k1 & 0xffffu), bf2f(k1 >> 16)};
+        if (NORM) {  // uniform: calls without in-kernel normalization skip the multiplies by 1
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { qf[e] *= rq[j]; kf[e] *= rk[j]; }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float fi = exp2_(d[j][e]), fj = exp2_(-d[j][e]);
+            kfi[j][e] = kf[e] * fi;
+            kfj[j][e] = kf[e] * fj;
+            qfi[j][e] = qf[e] * fi;
+        }
+    }
+}
+
 // V-major state rows of this lane: v = 16w + m, k = 16dt + 4g .. + 3
 __device__ __forceinline__ void store_state(float* dst, const f32x4 (&S)[8], int w, int g, int m) {
     float* row = dst + (16 * w + m) * D + 4 * g;
@@ -338,20 +553,19 @@ template <bool RG, bool P1, bool PREC>
 __global__ void __launch_bounds__(PF_THREADS, 1)
     chunk_kernel(PfParams p, const int32_t* __restrict__ tab, const int32_t* __restrict__ ck_idx, int list_off) {
     extern __shared__ __align__(16) unsigned char lds[];
-    float* sG = reinterpret_cast<float*>(lds + LDS_A);       // gate / Gamma, then k^ fi
-    float* sKA = sG;
+    float* sKA = reinterpret_cast<float*>(lds + LDS_A);      // k^ fi
     float* sQA = reinterpret_cast<float*>(lds + LDS_B);      // q^ fi
     half_t* sQt = reinterpret_cast<half_t*>(lds + LDS_B);    // Q~ (channels permuted)
     float* sKB = reinterpret_cast<float*>(lds + LDS_C);      // k^ fj
     half_t* sKd = reinterpret_cast<half_t*>(lds + LDS_C);    // Kd^T (tokens permuted)
     half_t* sW = reinterpret_cast<half_t*>(lds + LDS_BV);    // W (channels permuted), in region B's upper half
-    const uint16_t* sV = reinterpret_cast<const uint16_t*>(lds + LDS_W);  // this chunk's raw v rows (bf16)
+    uint16_t* sVt = reinterpret_cast<uint16_t*>(lds + LDS_VT);  // this chunk's raw v transposed (bf16)
     half_t* sAq = reinterpret_cast<half_t*>(lds + LDS_AQ);   // A_qk (columns permuted)
     half_t* sAk = reinterpret_cast<half_t*>(lds + LDS_AK);   // -A_kk off-diagonal blocks, T_II diagonal blocks
     float* sL = reinterpret_cast<float*>(lds + LDS_L);       // A_kk diagonal blocks, column-major [4][16][20]
     float* sF = reinterpret_cast<float*>(lds + LDS_F);       // per-channel factors [18][128]
-    float* sWt = reinterpret_cast<float*>(lds + LDS_WT);     // segment totals of the gate cumsum [4][128]
-    float* sGM = reinterpret_cast<float*>(lds + LDS_GM);     // the cumsum's block middle rows 16 I + 7 [4][128]
+    float* sWt = reinterpret_cast<float*>(lds + LDS_WT);     // gate totals of the 8 waves' rows [8][128]
+    half_t* sTl = reinterpret_cast<half_t*>(lds + LDS_WT);   // PREC: T_II's low parts [64][16], after the factors
     float* sBeta = reinterpret_cast<float*>(lds + LDS_BETA);
     float* sDT = reinterpret_cast<float*>(lds + LDS_DT);
 
@@ -427,7 +641,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     // ---- prologue.  Loads are issued in the order they are needed and none sits under a branch (the memory counter
     // completes in issue order, and a load on one path only makes the compiler wait for everything older): the first
     // chunk's rows (P0), the gate's dt_bias (P0), then the initial state, first used by the first walk.
-    int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4, r = tid >> 3, cb = tid & 7;
+    int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+    int c4 = lane & 31, row0 = 8 * w + 4 * (lane >> 5);  // the lane's channels 4 c4 .. + 3 and rows row0 .. + 3
     // The prologue's memory reads are issued in two dependent rounds: first what depends on the launch alone (the
     // table header, the chain entry, the gate's dt_bias, which is therefore waited for without waiting for the rows),
     // then what depends on the chain entry (the first chunk's rows, the pool row and its has_initial_state flag); the
@@ -438,9 +653,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     float dtb = RG ? p.dt_bias[cur.h * D + (tid & (D - 1))] : 0.f;
     asm volatile("" ::"s"(every), "s"(ws_arr), "s"(cur.ck_row0), "s"(cur.ck_single_raw), "s"(ck_words), "s"(cur.alog),
                  "s"(p.ws));
-    RawRow nx;
+    RawRows nx;
     // an empty sequence loads nothing
-    load_row<RG>(p, cur.h, cur.tstart, cur.nch > 0 ? min(64, cur.len) : 0, r, cb, RB, nx);
+    load_rows<RG>(p, cur.h, cur.tstart, cur.nch > 0 ? min(64, cur.len) : 0, row0, c4, RB, nx);
     f32x4 S[8];
     // initial state (lane: v = 16w + m, k = 16dt + 4g + e)
     auto load_start_state = [&](const float* src) {
@@ -466,7 +681,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     // A_qk blocks (0,1) and (2,3) are read by the walk and never written by the Gram phase
     for (int e = tid; e < 2 * 16 * 16; e += PF_THREADS) {
         const int b = e >> 8, ii = (e >> 4) & 15, jj = e & 15;
-        sAq[(32 * b + ii) * RS16S + 32 * b + pos32(16 + jj)] = (half_t)0.f;
+        sAq[half_at(32 * b + ii, 32 * b + pos32(16 + jj), RST, AQ_HALF)] = (half_t)0.f;
     }
     lds_barrier();  // sDT and the zeroed A_qk blocks are visible to every wave
 
@@ -516,153 +731,47 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             lane = tid & 63;
             m = lane & 15;
             g = lane >> 4;
-            r = tid >> 3;
-            cb = tid & 7;
+            c4 = lane & 31;
+            row0 = 8 * w + 4 * (lane >> 5);
             const int t0 = tstart + 64 * cl, L = min(64, len - 64 * cl);
             // the rows fetched during this chunk: the next chunk's, or during an item's last chunk the next item's
             // first
             const bool pf_here = cl + 1 < nch, pf = pf_here || more;
             const int pf_h = pf_here ? h : nx_h, pf_t = pf_here ? t0 + 64 : nx_t;
             const int pf_L = pf_here ? min(64, len - 64 * (cl + 1)) : (nx_nch > 0 ? min(64, nx_len) : 0);
-            // ================= P0: this chunk's raw rows (prefetched during the previous chunk)
-            // The raw q and k stay in registers until P2 (the next chunk's q, k loads reuse them from P5 on); the raw v
-            // goes to an LDS slot that only this thread reads back (the W area, which is free until P6), so its
-            // registers die here and the next chunk's v loads reuse them without a loop-carried copy.
-            *reinterpret_cast<u32x4*>(lds + LDS_W + r * (2 * RS16) + 32 * cb) = nx.v[0];
-            *reinterpret_cast<u32x4*>(lds + LDS_W + r * (2 * RS16) + 32 * cb + 16) = nx.v[1];
-            float gv[16];
-            if (RG) {
-                float rg[16];
-                const u32x4 gg[2] = {nx.g[0], nx.g[1]};
-                unpack16(gg, rg);
-                // g log2(e) = lb log2(e) sigmoid(e^{A_log} (x + dt_bias)), the sigmoid as 1 / (1 + 2^{An x + An dt})
-                // (one FMA, v_exp_f32, one add, v_rcp_f32), already in the log2 units of the cumsum.  Every row is
-                // computed; rows >= L get a zero multiplier (their raw gate reads as 0, so the sigmoid is finite): a
-                // computation under the row mask would branch per value and wait for every outstanding LDS read.
-                const float lbm = (r < L) ? p.lb * LOG2E : 0.f;
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    const f32x4 adt4 = *reinterpret_cast<const f32x4*>(&sDT[16 * cb + 4 * q4]);  // An dt_bias
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        gv[4 * q4 + e] = clamp_decay2(
-                            lbm * __builtin_amdgcn_rcpf(1.0f + exp2_(fmaf(An, rg[4 * q4 + e], adt4[e]))));
-                }
-            } else {  // natural-log units here; the cumsum scales them by log2(e) as it adds
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) gv[4 * i + j] = clamp_decay(__uint_as_float(nx.g[i][j]));
-            }
-            const float bx = RB ? sigmoid_rcp(bf2f(nx.beta)) : __uint_as_float(nx.beta);
-            const float bt = (r >= L) ? 0.f : bx;
-            float rq = 1.f, rk = 1.f;
-            if (NORM) {  // F.normalize(x, eps=1e-6) = x / max(|x|, 1e-6)  (kda/mi350x/reference.py:59-60)
-                // sums of squares straight from the packed bf16 pairs (v_dot2c_f32_bf16: the products are exact in
-                // fp32), so this phase unpacks no q / k value
-                float sq = 0.f, sk = 0.f;
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // element copies first: a bit cast of the vector element itself loses its index in this
-                        // compiler (every j read element 0)
-                        const uint32_t wq = nx.q[i][j], wk = nx.k[i][j];
-                        const bf16x2_t qp = __builtin_bit_cast(bf16x2_t, wq);
-                        const bf16x2_t kp = __builtin_bit_cast(bf16x2_t, wk);
-                        sq = __builtin_amdgcn_fdot2_f32_bf16(qp, qp, sq, false);
-                        sk = __builtin_amdgcn_fdot2_f32_bf16(kp, kp, sk, false);
-                    }
-                sq = sum8(sq);
-                sk = sum8(sk);
-                // 1 / max(|x|, 1e-6) = rsqrt(max(|x|^2, 1e-12)) through v_rsq_f32 (the IEEE sqrt is a sequence)
-                rq = __builtin_amdgcn_rsqf(fmaxf(sq, 1e-12f));
-                rk = __builtin_amdgcn_rsqf(fmaxf(sk, 1e-12f));
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<f32x4*>(&sG[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]) =
-                    f32x4{gv[4 * i], gv[4 * i + 1], gv[4 * i + 2], gv[4 * i + 3]};
-            if (cb == 0) sBeta[r] = bt;
+            // ================= P0-P2: the wave's rows to gated operands in registers (no barrier since the walk: what
+            // this writes to LDS the walk does not read), then, once every wave has left the walk, to regions A, B, C
+            f32x4 kfi[4], kfj[4], qfi[4];
+            chunk_front<RG>(nx, w, lane, L, RB, NORM, An, p.lb, sDT, sWt, sBeta, sVt, RS16S, kfi, kfj, qfi);
             lds_barrier();
-            // ================= P1: gate cumsum inside 16-row segments
-            {
-                const int c = tid & 127, s = tid >> 7;
-                float x[16];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) x[i] = sG[(16 * s + i) * RS32 + swz(c)];
-                if (RG) {  // already in log2 units
-#pragma unroll
-                    for (int i = 1; i < 16; ++i) x[i] += x[i - 1];
-                } else {  // natural log: the log2(e) scale goes into the adds
-                    x[0] *= LOG2E;
-#pragma unroll
-                    for (int i = 1; i < 16; ++i) x[i] = fmaf(x[i], LOG2E, x[i - 1]);
-                }
-#pragma unroll
-                for (int i = 0; i < 16; ++i) sG[(16 * s + i) * RS32 + swz(c)] = x[i];
-                sWt[s * 128 + c] = x[15];
-                sGM[s * 128 + c] = x[7];  // the factors' reference row of block s, kept apart so P2 can overwrite sG
-            }
-            lds_barrier();
-            // ================= P2: element factors (raw threads) and block factors (channel threads).  The block
-            // middle rows and segment totals come from sGM / sWt, so each raw thread reads only its own gate row from
-            // sG and can overwrite that row with k^ fi in place (no other thread reads it in this phase).
-            {
-                float qf[16], kf[16];
-                {
-                    const u32x4 a[2] = {nx.q[0], nx.q[1]}, b[2] = {nx.k[0], nx.k[1]};
-                    unpack16(a, qf);
-                    unpack16(b, kf);
-                }
-                if (NORM) {  // uniform: calls without in-kernel normalization skip the 32 multiplies by 1
-#pragma unroll
-                    for (int c = 0; c < 16; ++c) { kf[c] *= rk; qf[c] *= rq; }
-                }
-                const int I = r >> 4;
-                // block i of the row: its gate values are read before its k^ fi overwrites them (one thread, in order)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int o = r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1));
-                    const f32x4 a = *reinterpret_cast<const f32x4*>(&sG[o]);
-                    const f32x4 b = *reinterpret_cast<const f32x4*>(&sGM[I * 128 + 16 * cb + 4 * i]);
-                    f32x4 kfi, kfj, qfi;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int c = 4 * i + j;
-                        const float d = a[j] - b[j];  // Gamma_r - Gamma_m (the segment offset cancels)
-                        const float fi = exp2_(d), fj = exp2_(-d);
-                        kfi[j] = kf[c] * fi;
-                        kfj[j] = kf[c] * fj;
-                        qfi[j] = qf[c] * fi;
-                    }
-                    *reinterpret_cast<f32x4*>(&sQA[o]) = qfi;
-                    *reinterpret_cast<f32x4*>(&sKB[o]) = kfj;
-                    *reinterpret_cast<f32x4*>(&sKA[o]) = kfi;
-                }
+            for (int j = 0; j < 4; ++j) {
+                const int o = (row0 + j) * RS32 + 4 * c4;
+                *reinterpret_cast<f32x4*>(&sKA[o]) = kfi[j];
+                *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
+                *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
             }
             {
-                // qd is wave-uniform (128 threads per value): the row selection below branches on the scalar unit
+                // block factors, one thread per channel and factor group; qd is wave-uniform (128 threads per value):
+                // the row selection below branches on the scalar unit
                 const int c = tid & 127, qd = __builtin_amdgcn_readfirstlane(tid >> 7);
-                const float o1 = sWt[c], o2 = o1 + sWt[128 + c], o3 = o2 + sWt[256 + c];
-                // Gamma at rows 8 i + 7: block middles (sGM) and segment ends (sWt), plus the earlier segments
-                float gr[8];
+                float t[8];   // gate totals of rows 8 i .. 8 i + 7
+                float gr[8];  // Gamma at rows 8 i + 7
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float off = (i < 2) ? 0.f : (i < 4) ? o1 : (i < 6) ? o2 : o3;
-                    gr[i] = ((i & 1) ? sWt[(i >> 1) * 128 + c] : sGM[(i >> 1) * 128 + c]) + off;
-                }
+                for (int i = 0; i < 8; ++i) t[i] = sWt[i * 128 + c];
+                gr[0] = t[0];
+#pragma unroll
+                for (int i = 1; i < 8; ++i) gr[i] = gr[i - 1] + t[i];
 #pragma unroll
                 for (int f = 0; f < F_ROWS; ++f) {  // unrolled: gr[] is indexed by constants only (stays in registers)
                     if ((f & 3) != qd) continue;
                     float x;
                     if (f < F_B) {                       // a_I, I = f + 1: Gamma_m(I) - Gamma_{16I-1}
-                        const int I = f + 1;
-                        x = gr[2 * I] - gr[2 * I - 1];
+                        x = t[2 * (f + 1)];
                     } else if (f < F_X) {                // b_IJ
-                        const int t = f - F_B;
-                        const int I = t < 1 ? 1 : (t < 3 ? 2 : 3);
-                        const int J = t - (I * (I - 1)) / 2;
+                        const int u = f - F_B;
+                        const int I = u < 1 ? 1 : (u < 3 ? 2 : 3);
+                        const int J = u - (I * (I - 1)) / 2;
                         x = gr[2 * I - 1] - gr[2 * J];
                     } else if (f < F_Y) {
                         x = gr[2 * (f - F_X)];
@@ -671,7 +780,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     } else {
                         x = gr[7];
                     }
-                    sF[f * 128 + c] = exp2_(x);
+                    sF[f * RSF + f_at(c)] = exp2_(x);
                 }
             }
             lds_barrier();
@@ -681,13 +790,13 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 f32x4 akk = {0.f, 0.f, 0.f, 0.f}, aqk = akk;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const int c0 = 32 * s + 8 * g;
+                    const int c0 = gram_c0(s, g);
                     uint32_t kah[4], kal[4], qah[4], qal[4], kbh[4], kbl[4];  // bf16x8 fragments as 4 packed pairs
 #pragma unroll
                     for (int hf = 0; hf < 2; ++hf) {
-                        const f32x4 ka = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + swz(c0 + 4 * hf)]);
-                        const f32x4 qa = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + swz(c0 + 4 * hf)]);
-                        const f32x4 kb = *reinterpret_cast<const f32x4*>(&sKB[i * RS32 + swz(c0 + 4 * hf)]);
+                        const f32x4 ka = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + c0 + 4 * hf]);
+                        const f32x4 qa = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
+                        const f32x4 kb = *reinterpret_cast<const f32x4*>(&sKB[i * RS32 + c0 + 4 * hf]);
 #pragma unroll
                         for (int j = 0; j < 2; ++j) {
                             const int e = 2 * hf + j;
@@ -717,7 +826,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     lt[e] = (m < rr) ? bt4[e] * akk[e] : 0.f;
                     aq[e] = (half_t)((rr <= m) ? aqk[e] : 0.f);  // A_qk[16 I + m][16 I + rr], causal within the block
                 }
-                *reinterpret_cast<f16x4*>(&sAq[i * RS16S + pos64(16 * I + 4 * g)]) = aq;
+                *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * I + 4 * g), RST, AQ_HALF)]) = aq;
                 *reinterpret_cast<f32x4*>(&sL[(I * 16 + m) * 20 + 4 * g]) = lt;
                 // T_II = (I + L_II)^-1 of this wave's block while waves 4..7 still work on the off-diagonal blocks:
                 // lane j (every group of 16 lanes computes the same columns; lanes 0..15 write) solves column j by
@@ -744,10 +853,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         for (int ii = 0; ii < 16; ++ii) {
                             const half_t hi = (half_t)x[ii];
                             sAk[(16 * I + ii) * RS16S + 16 * I + m] = hi;
-                            // PREC: the low part in the A_qk block (I / 2, 2 + I % 2), a block of rows 0..31 and
-                            // columns 32..63 that the walk never reads and the Gram phase never writes
-                            if (PREC)
-                                sAq[(16 * (I >> 1) + ii) * RS16S + 32 + 16 * (I & 1) + m] = (half_t)(x[ii] - (float)hi);
+                            // PREC: the low part over the gate totals, which nothing reads until the next chunk's
+                            if (PREC) sTl[(16 * I + ii) * 16 + m] = (half_t)(x[ii] - (float)hi);
                         }
                     }
                 }
@@ -761,13 +868,13 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 for (int t = 0; t < 2; ++t) { akk[t] = f32x4{0.f, 0.f, 0.f, 0.f}; aqk[t] = akk[t]; }
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const int c0 = 32 * s + 8 * g;
+                    const int c0 = gram_c0(s, g);
                     f16x8 ka, qa;
 #pragma unroll
                     for (int hf = 0; hf < 2; ++hf) {
-                        const f32x4 a = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + swz(c0 + 4 * hf)]);
-                        const f32x4 q4 = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + swz(c0 + 4 * hf)]);
-                        const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[(F_A + I - 1) * 128 + c0 + 4 * hf]);
+                        const f32x4 a = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + c0 + 4 * hf]);
+                        const f32x4 q4 = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
+                        const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[(F_A + I - 1) * RSF + f_at(c0) + 4 * hf]);
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             ka[4 * hf + j] = (half_t)(a[j] * fa[j]);
@@ -782,8 +889,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                             f16x8 kb;
 #pragma unroll
                             for (int hf = 0; hf < 2; ++hf) {
-                                const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[jr * RS32 + swz(c0 + 4 * hf)]);
-                                const f32x4 fbv = *reinterpret_cast<const f32x4*>(&sF[fb * 128 + c0 + 4 * hf]);
+                                const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[jr * RS32 + c0 + 4 * hf]);
+                                const f32x4 fbv = *reinterpret_cast<const f32x4*>(&sF[fb * RSF + f_at(c0) + 4 * hf]);
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) kb[4 * hf + j] = (half_t)(b[j] * fbv[j]);
                             }
@@ -808,14 +915,10 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         *reinterpret_cast<f16x4*>(&sAk[i * RS16S + 16 * J + 4 * g]) = ak;
                         // PREC: the low part goes to the unused mirrored block (J, I) of the same array
                         if (PREC) *reinterpret_cast<f16x4*>(&sAk[(16 * J + m) * RS16S + 16 * I + 4 * g]) = al;
-                        *reinterpret_cast<f16x4*>(&sAq[i * RS16S + pos64(16 * J + 4 * g)]) = aq;
+                        *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * J + 4 * g), RST, AQ_HALF)]) = aq;
                     }
                 }
             }
-            // no barrier here: the reads below touch only the raw v staging and the thread's own q^ fi / k^ fj rows,
-            // which the Gram phase neither writes nor overwrites; the barrier before the layouts orders every Gram read
-            // of regions B and C before they are rewritten
-            // ================= P5: Q~, Kd^T, beta v into their walk layouts (raw threads)
             // The initial state loads (issued in the prologue or at the item's start) complete here, before any
             // next-chunk row is in flight: an empty use of S makes the compiler's wait for them fall at this point,
             // where in every later chunk only the long-finished output stores are outstanding, instead of before each
@@ -823,34 +926,27 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) asm volatile("" : "+v"(S[dt]));
             // the next chunk's q, k rows: issued here, consumed at the next P0 (their registers are free during P1..P4)
-            if (pf) load_row_qk(p, pf_h, pf_t, pf_L, r, cb, nx);
-            float qfi[16], kfj[16];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&sQA[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]);
-                const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) { qfi[4 * i + j] = a[j]; kfj[4 * i + j] = b[j]; }
-            }
+            if (pf) load_rows_qk(p, pf_h, pf_t, pf_L, row0, c4, nx);
             lds_barrier();  // regions B and C are rewritten below
             {
-                const int I = r >> 4;
-                const int hb = cb & 1, blk = cb >> 1;
+                // the lane still holds its rows' q^ fi and k^ fj; its block is I = w / 2
+                const f32x4 xf = *reinterpret_cast<const f32x4*>(&sF[(F_X + (w >> 1)) * RSF + f_at(4 * c4)]);
+                const f32x4 yf = *reinterpret_cast<const f32x4*>(&sF[(F_Y + (w >> 1)) * RSF + f_at(4 * c4)]);
+                const int qc = 32 * (c4 >> 3) + 8 * (c4 & 3) + (c4 & 4);  // stored position of channel 4 c4
 #pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    const f32x4 xf = *reinterpret_cast<const f32x4*>(&sF[(F_X + I) * 128 + 16 * cb + 4 * gq]);
+                for (int j = 0; j < 4; ++j) {
                     f16x4 o;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = (half_t)(qfi[4 * gq + e] * xf[e]);
-                    *reinterpret_cast<f16x4*>(&sQt[r * RS16 + 32 * blk + 8 * gq + 4 * hb]) = o;
+                    for (int e = 0; e < 4; ++e) o[e] = (half_t)(qfi[j][e] * xf[e]);
+                    *reinterpret_cast<f16x4*>(&sQt[(row0 + j) * RSQ + qc]) = o;
                 }
-                // Kd^T row of key channel k is stored at row 16 (k / 16) + (k % 16 ^ k / 16): the 8 channel blocks of a
-                // column write then land on 8 different banks
-                const int pr = pos64(r);
+                const int pr = pos64(row0);  // stored position of token row0 (row0 + 1 .. 3 follow it)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float y = sF[(F_Y + I) * 128 + 16 * cb + e];
-                    sKd[(16 * cb + (e ^ cb)) * RS16S + pr] = (half_t)(kfj[e] * y);
+                for (int e = 0; e < 4; ++e) {
+                    f16x4 o;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o[j] = (half_t)(kfj[j][e] * yf[e]);
+                    *reinterpret_cast<f16x4*>(&sKd[half_at(ch_row(4 * c4 + e), pr, RST, KD_HALF)]) = o;
                 }
             }
             // no barrier here: the solve reads k^ fi (region A), the raw v rows, -A_kk / T_II, the factors and beta,
@@ -858,7 +954,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             // operand reads before the layouts) passed the barrier above.  The walk reads the layouts after the solve's
             // barrier.
             // ================= P6: W and U by block forward substitution (wave w: channel / value tile w)
-            if (pf) load_row_vb(p, pf_h, pf_t, pf_L, r, cb, RB, nx);
+            if (pf) load_rows_vb(p, pf_h, pf_t, pf_L, row0, c4, RB, nx);
             f32x4 Ur[4];
             {
                 const int c = 16 * w + m;
@@ -871,14 +967,16 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 };
 #pragma unroll
                 for (int I = 0; I < 4; ++I) {
-                    const float xI = sF[(F_X + I) * 128 + c];
+                    const float xI = sF[(F_X + I) * RSF + f_at(16 * w) + m];
                     const f32x4 b4 = *reinterpret_cast<const f32x4*>(&sBeta[16 * I + 4 * g]);  // beta of the 4 rows
+                    // beta v straight from the raw v: 4 tokens of the lane's channel in one 8-byte read
+                    const u32x2 v4 = *reinterpret_cast<const u32x2*>(&sVt[(16 * w + (m ^ w)) * RS16S + 16 * I + 4 * g]);
+                    const float vf[4] = {bf2f(v4.x & 0xffffu), bf2f(v4.x >> 16), bf2f(v4.y & 0xffffu), bf2f(v4.y >> 16)};
                     f32x4 aw, au;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        const int rw = 16 * I + 4 * g + e;
-                        aw[e] = b4[e] * sKA[rw * RS32 + swz(c)] * xI;
-                        au[e] = b4[e] * bf2f(sV[rw * RS16 + c]);  // beta v straight from the raw v row
+                        aw[e] = b4[e] * sKA[(16 * I + 4 * g + e) * RS32 + c] * xI;
+                        au[e] = b4[e] * vf[e];
                     }
 #pragma unroll
                     for (int J = 0; J < I; ++J) {
@@ -899,31 +997,31 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     split4(aw, bwh, bwl);
                     split4(au, buh, bul);
                     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                    Xw[I] = mfma16(T, bwh, z);
+                    // W's tile transposed (swapped operands: the right-hand side's C layout is an A operand): the lane
+                    // holds 4 consecutive channels of token 16 I + m, one 8-byte store instead of 4 two-byte ones
+                    f32x4 Xt = mfma16(bwh, T, z);
+                    if (I < 3) Xw[I] = mfma16(T, bwh, z);
                     Ur[I] = mfma16(T, buh, z);
                     if (PREC) {
-                        const int tl = (16 * (I >> 1) + m) * RS16S + 32 + 16 * (I & 1) + 4 * g;
-                        const f16x4 Tl = *reinterpret_cast<const f16x4*>(&sAq[tl]);
-                        Xw[I] = mfma16(Tl, bwh, mfma16(T, bwl, Xw[I]));
+                        const f16x4 Tl = *reinterpret_cast<const f16x4*>(&sTl[(16 * I + m) * 16 + 4 * g]);
+                        Xt = mfma16(bwh, Tl, mfma16(bwl, T, Xt));
+                        if (I < 3) Xw[I] = mfma16(Tl, bwh, mfma16(T, bwl, Xw[I]));
                         Ur[I] = mfma16(Tl, buh, mfma16(T, bul, Ur[I]));
                     }
+                    *reinterpret_cast<f16x4*>(&sW[half_at(16 * I + m, 32 * (w >> 1) + 8 * g + 4 * (w & 1), RSW, W_HALF)]) =
+                        f16x4{(half_t)Xt[0], (half_t)Xt[1], (half_t)Xt[2], (half_t)Xt[3]};
                     if (I < 3) {
                         split4(Xw[I], Xh[I], Xl[I]);
                         split4(Ur[I], Uh[I], Ul[I]);
                     }
                 }
-                const int pc = 32 * (c >> 5) + pos32(c & 31);
-#pragma unroll
-                for (int I = 0; I < 4; ++I)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sW[(16 * I + 4 * g + e) * RS16 + pc] = (half_t)Xw[I][e];
             }
             // the next item's gate dt_bias for its first raw-row phase (this chunk's has read sDT; the barrier below
             // publishes the new values)
             if (RG && !pf_here && more && tid < D) sDT[tid] = dtb_next;
             lds_barrier();
             // ================= P7: the walk
-            if (pf) load_row_g<RG>(p, pf_h, pf_t, pf_L, r, cb, nx);
+            if (pf) load_rows_g<RG>(p, pf_h, pf_t, pf_L, row0, c4, nx);
             // every-n row 0 is the state before the sequence's first token: stored before the first walk changes S
             // (here rather than in the prologue, so that nothing before the first walk waits for the state loads)
             if (cl == 0 && ck_mode == 2 && every > 0 && first == 0) ck_store(ck_idx[ck_row0]);
@@ -945,7 +1043,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
                     for (int it = 0; it < 4; ++it) {
-                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sW[(16 * it + m) * RS16 + 32 * s + 8 * g]);
+                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sW[half_at(16 * it + m, 32 * s + 8 * g, RSW, W_HALF)]);
                         Vp[it] = mfma32(A, SB[s], Vp[it]);
                         Wp[it] = mfma32(A, PB[s], Wp[it]);
                     }
@@ -976,14 +1074,14 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acr = acc;
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
-                        const f16x8 B = *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RS16 + 32 * s + 8 * g]);
+                        const f16x8 B = *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RSQ + 32 * s + 8 * g]);
                         acc = mfma32(SB[s], B, acc);
                         acr = mfma32(PB[s], B, acr);
                     }
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
                         if (s <= (it >> 1)) {
-                            const f16x8 B = *reinterpret_cast<const f16x8*>(&sAq[(16 * it + m) * RS16S + 32 * s + 8 * g]);
+                            const f16x8 B = *reinterpret_cast<const f16x8*>(&sAq[half_at(16 * it + m, 32 * s + 8 * g, RST, AQ_HALF)]);
                             acc = mfma32(VB[s], B, acc);
                             acr = mfma32(WB[s], B, acr);
                         }
@@ -997,12 +1095,12 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 }
 #pragma unroll
                 for (int dt = 0; dt < 8; ++dt) {
-                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F_DEC * 128 + 16 * dt + 4 * g]);
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F_DEC * RSF + f_at(16 * dt) + 4 * g]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) { S[dt][e] *= d4[e]; Pm[dt][e] *= d4[e]; }
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
-                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[(16 * dt + (m ^ dt)) * RS16S + 32 * s + 8 * g]);
+                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[half_at(16 * dt + (m ^ dt), 32 * s + 8 * g, RST, KD_HALF)]);
                         S[dt] = mfma32(A, VB[s], S[dt]);
                         Pm[dt] = mfma32(A, WB[s], Pm[dt]);
                         if (PREC) {
@@ -1029,7 +1127,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
                     for (int it = 0; it < 4; ++it)
-                        Vp[it] = mfma32(*reinterpret_cast<const f16x8*>(&sW[(16 * it + m) * RS16 + 32 * s + 8 * g]), SB[s],
+                        Vp[it] = mfma32(*reinterpret_cast<const f16x8*>(&sW[half_at(16 * it + m, 32 * s + 8 * g, RSW, W_HALF)]), SB[s],
                                         Vp[it]);
 #pragma unroll
                 for (int it = 0; it < 4; ++it)
@@ -1056,13 +1154,13 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     for (int s = 0; s < 4; ++s)
 #pragma unroll
                         for (int it = 0; it < 4; ++it)
-                            ao[it] = mfma32(SB[s], *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RS16 + 32 * s + 8 * g]),
+                            ao[it] = mfma32(SB[s], *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RSQ + 32 * s + 8 * g]),
                                             ao[it]);
 #pragma unroll
                     for (int s = 0; s < 2; ++s)
 #pragma unroll
                         for (int it = 2 * s; it < 4; ++it)
-                            ao[it] = mfma32(VB[s], *reinterpret_cast<const f16x8*>(&sAq[(16 * it + m) * RS16S + 32 * s + 8 * g]),
+                            ao[it] = mfma32(VB[s], *reinterpret_cast<const f16x8*>(&sAq[half_at(16 * it + m, 32 * s + 8 * g, RST, AQ_HALF)]),
                                             ao[it]);
 #pragma unroll
                     for (int it = 0; it < 4; ++it) {
@@ -1075,12 +1173,12 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 }
 #pragma unroll
                 for (int dt = 0; dt < 8; ++dt) {
-                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F_DEC * 128 + 16 * dt + 4 * g]);
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F_DEC * RSF + f_at(16 * dt) + 4 * g]);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) S[dt][e] *= d4[e];
 #pragma unroll
                     for (int s = 0; s < 2; ++s) {
-                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[(16 * dt + (m ^ dt)) * RS16S + 32 * s + 8 * g]);
+                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[half_at(16 * dt + (m ^ dt), 32 * s + 8 * g, RST, KD_HALF)]);
                         S[dt] = mfma32(A, VB[s], S[dt]);
                         if (PREC) S[dt] = mfma32(A, VL[s], S[dt]);
                     }
@@ -1134,7 +1232,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
         const bool prefetched = nch > 0;
         cur = load_item(++kpos);
         if (!prefetched) {
-            load_row<RG>(p, cur.h, cur.tstart, cur.nch > 0 ? min(64, cur.len) : 0, r, cb, RB, nx);
+            load_rows<RG>(p, cur.h, cur.tstart, cur.nch > 0 ? min(64, cur.len) : 0, row0, c4, RB, nx);
             if (RG && threadIdx.x < D) sDT[threadIdx.x] = dtb_next;
             lds_barrier();
         }

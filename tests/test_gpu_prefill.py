@@ -311,6 +311,36 @@ def test_chunk_kda_gate_and_beta_in_kernel(oracle):
         assert rel_frob(f32(f1[n]), rf[n]) <= STATE_TOL, f"seq {n}"
 
 
+# lengths around the edges of the row groups a lane, a wave and a block own (4, 8, 16 rows) and of both chunk sizes
+_EDGE_LENS = [1, 3, 4, 5, 7, 8, 9, 12, 13, 15, 16, 17, 31, 32, 33, 47, 49, 55, 56, 57, 63, 64, 65, 68, 72, 73, 127, 129]
+
+
+@pytest.mark.parametrize("raw", [False, True], ids=["given", "raw"])
+@pytest.mark.parametrize("cus,chunk64", [(None, True), (4, True), (4, False)], ids=["whole", "lists", "chunk32"])
+def test_row_group_edges(oracle, raw, cus, chunk64):
+    """Sequences that end at, before and after every row-group edge, through each chunk kernel form with given and
+    in-kernel gates.  Bars as in the other parity tests: outputs 2e-2 x RMS beyond bf16 storage, states 1e-3."""
+    if not raw:
+        _plain_case(oracle, 2, _EDGE_LENS, 140, cus=cus, chunk64=chunk64)
+        return
+    kda = _kda()
+    H, lens = 2, _EDGE_LENS
+    _say(f"row group edges, gates in the kernel, cus={cus} chunk64={chunk64}")
+    g = gen(141)
+    q, k, v, raw_g, raw_b, A_log, dt_bias = _raw_inputs(g, sum(lens), H)
+    h0 = torch.randn(len(lens), H, D, D, generator=g) * 0.05
+    meta = _list_meta(kda, lens, H, cus, chunk64) if cus else None
+    o, fin = kda.kda_prefill(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), raw_g[None].to(DEV), raw_b[None].to(DEV),
+                             A_log.to(DEV), dt_bias.to(DEV), h0.to(DEV), torch.tensor(_cu(lens)).to(DEV), meta=meta)
+    torch.cuda.synchronize()
+    qn, kn, vf, gl, bt = _oracle_gated(oracle, q, k, v, raw_g, raw_b, A_log, dt_bias)
+    # the kernels raise log-decays below -9 to -9, which a one-token sequence's state shows (see the header)
+    ro, rf, _ = oracle.chains(qn, kn, vf, np.maximum(gl, -9.0), bt, _cu(lens), D ** -0.5, f32(h0), precision=64)
+    _check_out(o[0], ro, "row group edges", _cu(lens))
+    for n in range(len(lens)):
+        assert rel_frob(f32(fin[n]), rf[n]) <= STATE_TOL, f"seq {n} (len {lens[n]})"
+
+
 def _pages(slots, H, taps, g):
     """vLLM hybrid page layout (kda/mi350x/CONTRACT.md:60-67): conv state then SSM state per padded page."""
     dim = H * D
