@@ -10,30 +10,32 @@
 // model has it finish first, and launches in the precise mode keep chunk_kernel.
 //
 // Same algorithm, phases and operand conventions as chunk_kernel, with two row blocks of 16 instead of four:
-//   P0 raw rows (gate, beta, q / k sums of squares), P1 gate cumsum in 2 segments, P2 element and block factors
-//   (7 factor rows), P4 Gram tiles (wave I = 0 / 1: diagonal block I's A_kk with the bf16 hi / lo split, then T_II;
+//   P0-P2 rows to gated operands in registers (chunk_front), then the 7 block-factor rows, P4 Gram tiles (wave I = 0 / 1: diagonal block I's A_kk with the bf16 hi / lo split, then T_II;
 //   wave 2 + I: its A_qk, then one product of block (1, 0)), P5 Q~ and Kd^T layouts (tokens permuted by pos32),
 //   P6 W / U (wave w: channel / value tiles 2 w, 2 w + 1),
 //   P7 the walk (wave w: S[:, 32 w .. 32 w + 31], K step outermost).  Checkpoints fall on 64-token boundaries, i.e.
 //   after every second chunk (or after the last chunk of the sequence).
 constexpr int C32_THREADS = 256;
-constexpr int RS16T = 40;                                // fp16 rows of 32 (+ 8)
-constexpr int C32_A = 0;                                 // gate / Gamma, then k^ fi: fp32 [32][RS32]
-constexpr int C32_B = C32_A + 32 * RS32 * 4;             // q^ fi fp32 [32][RS32]; then Q~ fp16 [32][RS16]
-constexpr int C32_BV = C32_B + 32 * RS16 * 2;            // W fp16 [32][RS16] (region B's upper half)
-constexpr int C32_C = C32_B + 2 * 32 * RS16 * 2;         // k^ fj fp32 [32][RS32]; then Kd^T fp16 [128][RS16T]
-constexpr int C32_V = C32_C + 32 * RS32 * 4;             // raw v rows bf16 [32][RS16]
-constexpr int C32_AQ = C32_V + 32 * RS16 * 2;            // A_qk fp16 [32][RS16T] (columns permuted)
-constexpr int C32_AK = C32_AQ + 32 * RS16T * 2;          // -A_kk block (1, 0) and T_II diagonal blocks fp16 [32][RS16T]
-constexpr int C32_GM = C32_AK + 32 * RS16T * 2;          // the cumsum's block middle rows [2][128] fp32
-constexpr int C32_F = C32_GM + 2 * 128 * 4;              // factor rows [7][128] fp32
-constexpr int C32_WT = C32_F + 7 * 128 * 4;              // segment totals [2][128] fp32
-constexpr int C32_BETA = C32_WT + 2 * 128 * 4;           // [32] fp32
+constexpr int RST32 = 48;                                // rows of 32 tokens (fp16): 6 slots, no conflicts (see RST)
+constexpr int RSV32 = 40;                                // V^T rows (bf16, 32 tokens)
+constexpr int RSA32 = 40;                                // -A_kk / T_II rows
+constexpr int W_HALF32 = 32 * RSW;                       // elements of a half array of W
+constexpr int C32_A = 0;                                 // k^ fi: fp32 [32][RS32]
+constexpr int C32_B = C32_A + 32 * RS32 * 4;             // q^ fi fp32 [32][RS32]; then Q~ fp16 [32][RSQ]
+constexpr int C32_BV = C32_B + 32 * RSQ * 2;             // W fp16 [2][32][RSW] (region B's upper half)
+constexpr int C32_C = C32_BV + 2 * W_HALF32 * 2;         // k^ fj fp32 [32][RS32]; then Kd^T fp16 [128][RST32]
+constexpr int C32_VT = C32_C + 32 * RS32 * 4;            // V^T bf16 [128][RSV32]
+constexpr int C32_AQ = C32_VT + 128 * RSV32 * 2;         // A_qk fp16 [32][RST32] (columns permuted)
+constexpr int C32_AK = C32_AQ + 32 * RST32 * 2;          // -A_kk block (1, 0) and T_II diagonal blocks fp16 [32][RSA32]
+constexpr int C32_F = C32_AK + 32 * RSA32 * 2;           // factor rows [7][RSF] fp32
+constexpr int C32_WT = C32_F + 7 * RSF * 4;              // gate totals of the 4 waves' rows [4][128] fp32
+constexpr int C32_BETA = C32_WT + 4 * 128 * 4;           // [32] fp32
 constexpr int C32_DT = C32_BETA + 32 * 4;                // An dt_bias [128] fp32 (gate in the kernel)
 constexpr int C32_L = C32_DT + 128 * 4;                  // A_kk diagonal blocks, column-major [2][16][20] fp32
 constexpr int C32_TOTAL = C32_L + 2 * 16 * 20 * 4;
-static_assert(32 * RS32 * 4 <= 2 * 32 * RS16 * 2, "q^ fi fits region B");
-static_assert(128 * RS16T * 2 <= 32 * RS32 * 4, "Kd^T fits region C");
+static_assert(32 * RS32 * 4 <= 32 * RSQ * 2 + 2 * W_HALF32 * 2, "q^ fi fits region B");
+static_assert(128 * RST32 * 2 <= 32 * RS32 * 4, "Kd^T fits region C");
+static_assert(W_HALF32 * 2 % 256 == 0, "half arrays share their banks");
 static_assert(2 * C32_TOTAL <= 160 * 1024, "two workgroups per CU");
 // factor rows: a_1 = e^{Gamma_m(1) - Gamma_15}, b_10 = e^{Gamma_15 - Gamma_m(0)}, x_I = e^{Gamma_m(I)},
 // y_I = e^{Gamma_c - Gamma_m(I)}, e^{Gamma_c} (Gamma_m(I): the middle row 16 I + 7 of block I; Gamma_c: the last row)
@@ -63,20 +65,18 @@ template <bool RG>
 __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     chunk32_kernel(PfParams p, const int32_t* __restrict__ tab, const int32_t* __restrict__ ck_idx, int list_off) {
     extern __shared__ __align__(16) unsigned char lds[];
-    float* sG = reinterpret_cast<float*>(lds + C32_A);
-    float* sKA = sG;
+    float* sKA = reinterpret_cast<float*>(lds + C32_A);
     float* sQA = reinterpret_cast<float*>(lds + C32_B);
     half_t* sQt = reinterpret_cast<half_t*>(lds + C32_B);
     half_t* sW = reinterpret_cast<half_t*>(lds + C32_BV);
     float* sKB = reinterpret_cast<float*>(lds + C32_C);
     half_t* sKd = reinterpret_cast<half_t*>(lds + C32_C);
-    const uint16_t* sV = reinterpret_cast<const uint16_t*>(lds + C32_V);
+    uint16_t* sVt = reinterpret_cast<uint16_t*>(lds + C32_VT);
     half_t* sAq = reinterpret_cast<half_t*>(lds + C32_AQ);
     half_t* sAk = reinterpret_cast<half_t*>(lds + C32_AK);
     float* sL = reinterpret_cast<float*>(lds + C32_L);
     float* sF = reinterpret_cast<float*>(lds + C32_F);
     float* sWt = reinterpret_cast<float*>(lds + C32_WT);
-    float* sGM = reinterpret_cast<float*>(lds + C32_GM);
     float* sBeta = reinterpret_cast<float*>(lds + C32_BETA);
     float* sDT = reinterpret_cast<float*>(lds + C32_DT);
 
@@ -105,11 +105,12 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
     } else {
         src = p.init_state ? p.init_state + ((int64_t)n * H + h) * D * D : nullptr;
     }
-    int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4, r = tid >> 3, cb = tid & 7;
+    int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+    int c4 = lane & 31, row0 = 8 * w + 4 * (lane >> 5);  // the lane's channels 4 c4 .. + 3 and rows row0 .. + 3
     const float dtb = RG ? p.dt_bias[h * D + (tid & (D - 1))] : 0.f;
     const float alog = RG ? p.A_log[h] : 0.f;
-    RawRow nx;
-    load_row<RG>(p, h, tstart, nch > 0 ? min(32, len) : 0, r, cb, RB, nx);  // an empty sequence loads nothing
+    RawRows nx;
+    load_rows<RG>(p, h, tstart, nch > 0 ? min(32, len) : 0, row0, c4, RB, nx);  // an empty sequence loads nothing
     f32x4 S[8][2];
     {
         // through a descriptor of no records when there is no start state; base and size wave-uniform
@@ -137,7 +138,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
         if (tid < D) sDT[tid] = An * dtb;
     }
     // A_qk block (0, 1) is read by the walk and never written by the Gram phase
-    sAq[(tid >> 4) * RS16T + pos32(16 + (tid & 15))] = (half_t)0.f;
+    sAq[(tid >> 4) * RST32 + pos32(16 + (tid & 15))] = (half_t)0.f;
     lds_barrier();
 
     for (int cl = 0; cl < nch; ++cl) {
@@ -147,127 +148,38 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
         lane = tid & 63;
         m = lane & 15;
         g = lane >> 4;
-        r = tid >> 3;
-        cb = tid & 7;
+        c4 = lane & 31;
+        row0 = 8 * w + 4 * (lane >> 5);
         const int t0 = tstart + 32 * cl, L = min(32, len - 32 * cl);
         const bool pf = cl + 1 < nch;
         const int pf_t = t0 + 32, pf_L = pf ? min(32, len - 32 * (cl + 1)) : 0;
-        // ================= P0: raw rows (v to LDS; gate, beta; q / k sums of squares)
-        *reinterpret_cast<u32x4*>(lds + C32_V + r * (2 * RS16) + 32 * cb) = nx.v[0];
-        *reinterpret_cast<u32x4*>(lds + C32_V + r * (2 * RS16) + 32 * cb + 16) = nx.v[1];
-        float gv[16];
-        if (RG) {
-            float rg[16];
-            const u32x4 gg[2] = {nx.g[0], nx.g[1]};
-            unpack16(gg, rg);
-            const float lbm = (r < L) ? p.lb * LOG2E : 0.f;
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const f32x4 adt4 = *reinterpret_cast<const f32x4*>(&sDT[16 * cb + 4 * q4]);
-#pragma unroll
-                for (int ee = 0; ee < 4; ++ee)
-                    gv[4 * q4 + ee] =
-                        clamp_decay2(lbm * __builtin_amdgcn_rcpf(1.0f + exp2_(fmaf(An, rg[4 * q4 + ee], adt4[ee]))));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) gv[4 * i + j] = clamp_decay(__uint_as_float(nx.g[i][j]));
-        }
-        const float bx = RB ? sigmoid_rcp(bf2f(nx.beta)) : __uint_as_float(nx.beta);
-        const float bt = (r >= L) ? 0.f : bx;
-        float rq = 1.f, rk = 1.f;
-        if (NORM) {  // F.normalize(x, eps=1e-6)  (kda/mi350x/reference.py:59-60)
-            float sq = 0.f, sk = 0.f;
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t wq = nx.q[i][j], wk = nx.k[i][j];  // element copies (see chunk_kernel)
-                    const bf16x2_t qp = __builtin_bit_cast(bf16x2_t, wq);
-                    const bf16x2_t kp = __builtin_bit_cast(bf16x2_t, wk);
-                    sq = __builtin_amdgcn_fdot2_f32_bf16(qp, qp, sq, false);
-                    sk = __builtin_amdgcn_fdot2_f32_bf16(kp, kp, sk, false);
-                }
-            sq = sum8(sq);
-            sk = sum8(sk);
-            rq = __builtin_amdgcn_rsqf(fmaxf(sq, 1e-12f));
-            rk = __builtin_amdgcn_rsqf(fmaxf(sk, 1e-12f));
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<f32x4*>(&sG[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]) =
-                f32x4{gv[4 * i], gv[4 * i + 1], gv[4 * i + 2], gv[4 * i + 3]};
-        if (cb == 0) sBeta[r] = bt;
-        lds_barrier();
-        // ================= P1: gate cumsum inside the 2 segments of 16 rows
+        // ================= P0-P2: the wave's rows to gated operands in registers, then to regions A, B, C; block factors
         {
-            const int c = tid & 127, s = tid >> 7;
-            float x[16];
+            f32x4 kfi[4], kfj[4], qfi[4];
+            chunk_front<RG>(nx, w, lane, L, RB, NORM, An, p.lb, sDT, sWt, sBeta, sVt, RSV32, kfi, kfj, qfi);
+            lds_barrier();
 #pragma unroll
-            for (int i = 0; i < 16; ++i) x[i] = sG[(16 * s + i) * RS32 + swz(c)];
-            if (RG) {
-#pragma unroll
-                for (int i = 1; i < 16; ++i) x[i] += x[i - 1];
-            } else {
-                x[0] *= LOG2E;
-#pragma unroll
-                for (int i = 1; i < 16; ++i) x[i] = fmaf(x[i], LOG2E, x[i - 1]);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) sG[(16 * s + i) * RS32 + swz(c)] = x[i];
-            sWt[s * 128 + c] = x[15];
-            sGM[s * 128 + c] = x[7];
-        }
-        lds_barrier();
-        // ================= P2: element factors (raw threads) and the 7 block-factor rows (channel threads)
-        {
-            float qf[16], kf[16];
-            {
-                const u32x4 a[2] = {nx.q[0], nx.q[1]}, b[2] = {nx.k[0], nx.k[1]};
-                unpack16(a, qf);
-                unpack16(b, kf);
-            }
-            if (NORM) {
-#pragma unroll
-                for (int c = 0; c < 16; ++c) { kf[c] *= rk; qf[c] *= rq; }
-            }
-            const int I = r >> 4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int o = r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1));
-                const f32x4 a = *reinterpret_cast<const f32x4*>(&sG[o]);
-                const f32x4 b = *reinterpret_cast<const f32x4*>(&sGM[I * 128 + 16 * cb + 4 * i]);
-                f32x4 kfi, kfj, qfi;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int c = 4 * i + j;
-                    const float d = a[j] - b[j];
-                    const float fi = exp2_(d), fj = exp2_(-d);
-                    kfi[j] = kf[c] * fi;
-                    kfj[j] = kf[c] * fj;
-                    qfi[j] = qf[c] * fi;
-                }
-                *reinterpret_cast<f32x4*>(&sQA[o]) = qfi;
-                *reinterpret_cast<f32x4*>(&sKB[o]) = kfj;
-                *reinterpret_cast<f32x4*>(&sKA[o]) = kfi;
+            for (int j = 0; j < 4; ++j) {
+                const int o = (row0 + j) * RS32 + 4 * c4;
+                *reinterpret_cast<f32x4*>(&sKA[o]) = kfi[j];
+                *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
+                *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
             }
         }
         {
             const int c = tid & 127, qd = __builtin_amdgcn_readfirstlane(tid >> 7);  // wave-uniform
-            const float o1 = sWt[c];
-            // Gamma at rows 7, 15, 23, 31
-            const float gr0 = sGM[c], gr1 = o1, gr2 = sGM[128 + c] + o1, gr3 = sWt[128 + c] + o1;
+            const int fc = f_at(c);
+            // gate totals of rows 8 i .. 8 i + 7; Gamma at rows 7, 15, 23, 31 are their running sums
+            const float t0 = sWt[c], t1 = sWt[128 + c], t2 = sWt[256 + c], t3 = sWt[384 + c];
             if (qd == 0) {
-                sF[F32_A * 128 + c] = exp2_(gr2 - gr1);
-                sF[F32_X * 128 + c] = exp2_(gr0);
-                sF[(F32_Y + 1) * 128 + c] = exp2_(gr3 - gr2);
-                sF[F32_DEC * 128 + c] = exp2_(gr3);
+                sF[F32_A * RSF + fc] = exp2_(t2);
+                sF[F32_X * RSF + fc] = exp2_(t0);
+                sF[(F32_Y + 1) * RSF + fc] = exp2_(t3);
+                sF[F32_DEC * RSF + fc] = exp2_((t0 + t1) + (t2 + t3));
             } else {
-                sF[F32_B * 128 + c] = exp2_(gr1 - gr0);
-                sF[(F32_X + 1) * 128 + c] = exp2_(gr2);
-                sF[F32_Y * 128 + c] = exp2_(gr3 - gr0);
+                sF[F32_B * RSF + fc] = exp2_(t1);
+                sF[(F32_X + 1) * RSF + fc] = exp2_((t0 + t1) + t2);
+                sF[F32_Y * RSF + fc] = exp2_(t1 + (t2 + t3));
             }
         }
         lds_barrier();
@@ -281,12 +193,12 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             const float* sX = kk ? sKA : sQA;  // the product's second operand: k^ fi (A_kk) or q^ fi (A_qk)
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const int c0 = 32 * s + 8 * g;
+                const int c0 = gram_c0(s, g);
                 uint32_t xh[4], xl[4], kbh[4], kbl[4];
 #pragma unroll
                 for (int hf = 0; hf < 2; ++hf) {
-                    const f32x4 xa = *reinterpret_cast<const f32x4*>(&sX[i * RS32 + swz(c0 + 4 * hf)]);
-                    const f32x4 kb = *reinterpret_cast<const f32x4*>(&sKB[i * RS32 + swz(c0 + 4 * hf)]);
+                    const f32x4 xa = *reinterpret_cast<const f32x4*>(&sX[i * RS32 + c0 + 4 * hf]);
+                    const f32x4 kb = *reinterpret_cast<const f32x4*>(&sKB[i * RS32 + c0 + 4 * hf]);
 #pragma unroll
                     for (int j = 0; j < 2; ++j) {
                         const int ee = 2 * hf + j;
@@ -328,13 +240,13 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                 }
                 if (g == 0) {
 #pragma unroll
-                    for (int ii = 0; ii < 16; ++ii) sAk[(16 * I + ii) * RS16T + 16 * I + m] = (half_t)x[ii];
+                    for (int ii = 0; ii < 16; ++ii) sAk[(16 * I + ii) * RSA32 + 16 * I + m] = (half_t)x[ii];
                 }
             } else {
                 f16x4 aq;
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) aq[ee] = (half_t)((4 * g + ee <= m) ? acc[ee] : 0.f);  // causal
-                *reinterpret_cast<f16x4*>(&sAq[i * RS16T + pos32(16 * I + 4 * g)]) = aq;
+                *reinterpret_cast<f16x4*>(&sAq[i * RST32 + pos32(16 * I + 4 * g)]) = aq;
             }
         }
         if (w >= 2) {  // block (1, 0): wave 2 A_kk, wave 3 A_qk (transposed tiles: lane (g, m) holds row 16 + m,
@@ -345,14 +257,14 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const int c0 = 32 * s + 8 * g;
+                const int c0 = gram_c0(s, g);
                 f16x8 xa, kb;
 #pragma unroll
                 for (int hf = 0; hf < 2; ++hf) {
-                    const f32x4 a = *reinterpret_cast<const f32x4*>(&sX[i * RS32 + swz(c0 + 4 * hf)]);
-                    const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[F32_A * 128 + c0 + 4 * hf]);
-                    const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[m * RS32 + swz(c0 + 4 * hf)]);
-                    const f32x4 fb = *reinterpret_cast<const f32x4*>(&sF[F32_B * 128 + c0 + 4 * hf]);
+                    const f32x4 a = *reinterpret_cast<const f32x4*>(&sX[i * RS32 + c0 + 4 * hf]);
+                    const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[F32_A * RSF + f_at(c0) + 4 * hf]);
+                    const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[m * RS32 + c0 + 4 * hf]);
+                    const f32x4 fb = *reinterpret_cast<const f32x4*>(&sF[F32_B * RSF + f_at(c0) + 4 * hf]);
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         xa[4 * hf + j] = (half_t)(a[j] * fa[j]);
@@ -366,93 +278,93 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                 f16x4 ak;
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) ak[ee] = (half_t)(nb * acc[ee]);
-                *reinterpret_cast<f16x4*>(&sAk[i * RS16T + 4 * g]) = ak;
+                *reinterpret_cast<f16x4*>(&sAk[i * RSA32 + 4 * g]) = ak;
             } else {
                 f16x4 aq;
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) aq[ee] = (half_t)acc[ee];
-                *reinterpret_cast<f16x4*>(&sAq[i * RS16T + pos32(4 * g)]) = aq;
+                *reinterpret_cast<f16x4*>(&sAq[i * RST32 + pos32(4 * g)]) = aq;
             }
         }
-        // ================= P5: Q~, Kd^T into their walk layouts (raw threads)
+        // ================= P5: Q~, Kd^T into their walk layouts (the lane's rows)
         // the start state's loads complete here in the first chunk (an empty use of S), not before a later walk
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct) asm volatile("" : "+v"(S[dt][ct]));
-        if (pf) load_row_qk(p, h, pf_t, pf_L, r, cb, nx);
-        float qfi[16], kfj[16];
+        if (pf) load_rows_qk(p, h, pf_t, pf_L, row0, c4, nx);
+        // the lane's q^ fi and k^ fj back from LDS: with 64 registers of S, holding their 32 through the Gram phase spills
+        f32x4 kfj[4], qfi[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(&sQA[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]);
-            const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[r * RS32 + 16 * cb + 4 * (i ^ (cb >> 1))]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { qfi[4 * i + j] = a[j]; kfj[4 * i + j] = b[j]; }
+        for (int j = 0; j < 4; ++j) {
+            qfi[j] = *reinterpret_cast<const f32x4*>(&sQA[(row0 + j) * RS32 + 4 * c4]);
+            kfj[j] = *reinterpret_cast<const f32x4*>(&sKB[(row0 + j) * RS32 + 4 * c4]);
         }
         lds_barrier();  // regions B and C are rewritten below
         {
-            const int I = r >> 4;
-            const int hb = cb & 1, blk = cb >> 1;
+            const f32x4 xf = *reinterpret_cast<const f32x4*>(&sF[(F32_X + (w >> 1)) * RSF + f_at(4 * c4)]);
+            const f32x4 yf = *reinterpret_cast<const f32x4*>(&sF[(F32_Y + (w >> 1)) * RSF + f_at(4 * c4)]);
+            const int qc = 32 * (c4 >> 3) + 8 * (c4 & 3) + (c4 & 4);  // stored position of channel 4 c4
 #pragma unroll
-            for (int gq = 0; gq < 4; ++gq) {
-                const f32x4 xf = *reinterpret_cast<const f32x4*>(&sF[(F32_X + I) * 128 + 16 * cb + 4 * gq]);
+            for (int j = 0; j < 4; ++j) {
                 f16x4 o;
 #pragma unroll
-                for (int ee = 0; ee < 4; ++ee) o[ee] = (half_t)(qfi[4 * gq + ee] * xf[ee]);
-                *reinterpret_cast<f16x4*>(&sQt[r * RS16 + 32 * blk + 8 * gq + 4 * hb]) = o;
+                for (int ee = 0; ee < 4; ++ee) o[ee] = (half_t)(qfi[j][ee] * xf[ee]);
+                *reinterpret_cast<f16x4*>(&sQt[(row0 + j) * RSQ + qc]) = o;
             }
-            const int pr = pos32(r);
+            const int pr = pos32(row0);  // stored position of token row0 (row0 + 1 .. 3 follow it)
 #pragma unroll
-            for (int ee = 0; ee < 16; ++ee) {
-                const float y = sF[(F32_Y + I) * 128 + 16 * cb + ee];
-                sKd[(16 * cb + (ee ^ cb)) * RS16T + pr] = (half_t)(kfj[ee] * y);
+            for (int ee = 0; ee < 4; ++ee) {
+                f16x4 o;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o[j] = (half_t)(kfj[j][ee] * yf[ee]);
+                *reinterpret_cast<f16x4*>(&sKd[ch_row(4 * c4 + ee) * RST32 + pr]) = o;
             }
         }
         // ================= P6: W and U by block forward substitution (wave w: channel / value tiles 2 w, 2 w + 1)
-        if (pf) load_row_vb(p, h, pf_t, pf_L, r, cb, RB, nx);
+        if (pf) load_rows_vb(p, h, pf_t, pf_L, row0, c4, RB, nx);
         f32x4 Ur[2][2];  // [block I][tile t]: U[token 16 I + 4 g + e][value 32 w + 16 t + m]
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const int c = 16 * (2 * w + t) + m;
-            f32x4 Xw[2];
+            const int tw = 2 * w + t, c = 16 * tw + m;
             f16x4 Xh0, Uh0;
 #pragma unroll
             for (int I = 0; I < 2; ++I) {
-                const float xI = sF[(F32_X + I) * 128 + c];
+                const float xI = sF[(F32_X + I) * RSF + f_at(16 * tw) + m];
                 const f32x4 b4 = *reinterpret_cast<const f32x4*>(&sBeta[16 * I + 4 * g]);
+                const u32x2 v4 = *reinterpret_cast<const u32x2*>(&sVt[(16 * tw + (m ^ tw)) * RSV32 + 16 * I + 4 * g]);
+                const float vf[4] = {bf2f(v4.x & 0xffffu), bf2f(v4.x >> 16), bf2f(v4.y & 0xffffu), bf2f(v4.y >> 16)};
                 f32x4 aw, au;
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) {
-                    const int rw = 16 * I + 4 * g + ee;
-                    aw[ee] = b4[ee] * sKA[rw * RS32 + swz(c)] * xI;
-                    au[ee] = b4[ee] * bf2f(sV[rw * RS16 + c]);
+                    aw[ee] = b4[ee] * sKA[(16 * I + 4 * g + ee) * RS32 + c] * xI;
+                    au[ee] = b4[ee] * vf[ee];
                 }
                 if (I == 1) {
-                    const f16x4 A = *reinterpret_cast<const f16x4*>(&sAk[(16 + m) * RS16T + 4 * g]);
+                    const f16x4 A = *reinterpret_cast<const f16x4*>(&sAk[(16 + m) * RSA32 + 4 * g]);
                     aw = mfma16(A, Xh0, aw);
                     au = mfma16(A, Uh0, au);
                 }
-                const f16x4 T = *reinterpret_cast<const f16x4*>(&sAk[(16 * I + m) * RS16T + 16 * I + 4 * g]);
+                const f16x4 T = *reinterpret_cast<const f16x4*>(&sAk[(16 * I + m) * RSA32 + 16 * I + 4 * g]);
                 f16x4 bwh, buh;
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) { bwh[ee] = (half_t)aw[ee]; buh[ee] = (half_t)au[ee]; }
                 const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                Xw[I] = mfma16(T, bwh, z);
+                // W's tile transposed (see chunk_kernel): 4 consecutive channels of token 16 I + m per lane
+                const f32x4 Xt = mfma16(bwh, T, z);
                 Ur[I][t] = mfma16(T, buh, z);
+                *reinterpret_cast<f16x4*>(&sW[half_at(16 * I + m, 32 * w + 8 * g + 4 * t, RSW, W_HALF32)]) =
+                    f16x4{(half_t)Xt[0], (half_t)Xt[1], (half_t)Xt[2], (half_t)Xt[3]};
                 if (I == 0) {
+                    const f32x4 Xw = mfma16(T, bwh, z);
 #pragma unroll
-                    for (int ee = 0; ee < 4; ++ee) { Xh0[ee] = (half_t)Xw[0][ee]; Uh0[ee] = (half_t)Ur[0][t][ee]; }
+                    for (int ee = 0; ee < 4; ++ee) { Xh0[ee] = (half_t)Xw[ee]; Uh0[ee] = (half_t)Ur[0][t][ee]; }
                 }
             }
-            const int pc = 32 * (c >> 5) + pos32(c & 31);
-#pragma unroll
-            for (int I = 0; I < 2; ++I)
-#pragma unroll
-                for (int ee = 0; ee < 4; ++ee) sW[(16 * I + 4 * g + ee) * RS16 + pc] = (half_t)Xw[I][ee];
         }
         lds_barrier();
         // ================= P7: the walk (wave w: S[:, 32 w .. 32 w + 31])
-        if (pf) load_row_g<RG>(p, h, pf_t, pf_L, r, cb, nx);
+        if (pf) load_rows_g<RG>(p, h, pf_t, pf_L, row0, c4, nx);
         // every-n row 0: the state before the sequence's first token
         if (cl == 0 && ck_mode == 2 && every > 0 && first == 0) ck_store(ck_idx[ck_row0]);
         {
@@ -475,7 +387,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int it = 0; it < 2; ++it) {
-                    const f16x8 A = *reinterpret_cast<const f16x8*>(&sW[(16 * it + m) * RS16 + 32 * s + 8 * g]);
+                    const f16x8 A = *reinterpret_cast<const f16x8*>(&sW[half_at(16 * it + m, 32 * s + 8 * g, RSW, W_HALF32)]);
 #pragma unroll
                     for (int ct = 0; ct < 2; ++ct) Vp[it][ct] = mfma32(A, SB[s][ct], Vp[it][ct]);
                 }
@@ -497,13 +409,13 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int it = 0; it < 2; ++it) {
-                    const f16x8 B = *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RS16 + 32 * s + 8 * g]);
+                    const f16x8 B = *reinterpret_cast<const f16x8*>(&sQt[(16 * it + m) * RSQ + 32 * s + 8 * g]);
 #pragma unroll
                     for (int ct = 0; ct < 2; ++ct) ao[it][ct] = mfma32(SB[s][ct], B, ao[it][ct]);
                 }
 #pragma unroll
             for (int it = 0; it < 2; ++it) {
-                const f16x8 B = *reinterpret_cast<const f16x8*>(&sAq[(16 * it + m) * RS16T + 8 * g]);
+                const f16x8 B = *reinterpret_cast<const f16x8*>(&sAq[(16 * it + m) * RST32 + 8 * g]);
 #pragma unroll
                 for (int ct = 0; ct < 2; ++ct) ao[it][ct] = mfma32(VB[ct], B, ao[it][ct]);
             }
@@ -520,8 +432,8 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             // S <- diag(e^{Gamma_c}) S + Kd^T V'
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
-                const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F32_DEC * 128 + 16 * dt + 4 * g]);
-                const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[(16 * dt + (m ^ dt)) * RS16T + 8 * g]);
+                const f32x4 d4 = *reinterpret_cast<const f32x4*>(&sF[F32_DEC * RSF + f_at(16 * dt) + 4 * g]);
+                const f16x8 A = *reinterpret_cast<const f16x8*>(&sKd[(16 * dt + (m ^ dt)) * RST32 + 8 * g]);
 #pragma unroll
                 for (int ct = 0; ct < 2; ++ct) {
 #pragma unroll

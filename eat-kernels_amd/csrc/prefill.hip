@@ -64,7 +64,6 @@ constexpr int RS32 = 132;   // fp32 rows of 128
 constexpr int RSQ = 144;    // Q~ rows (fp16)
 constexpr int RSW = 72;     // rows of a half array of W (fp16, 64 channels)
 constexpr int RST = 40;     // rows of a half array of A_qk or Kd^T (fp16, 32 tokens)
-constexpr int RS16 = 136;   // fp16 rows of 128
 constexpr int RS16S = 72;   // fp16 rows of 64
 constexpr int RSF = 132;    // factor rows: channel c at c + 4 (c / 64) (see f_at)
 constexpr int W_HALF = 64 * RSW, AQ_HALF = 64 * RST, KD_HALF = 128 * RST;  // elements of a half array
@@ -139,11 +138,6 @@ __device__ __forceinline__ int gram_c0(int s, int g) { return 64 * (g & 1) + 32 
 // channel c in a factor row: the two 64-channel halves sit 4 floats apart in the banks, so that the lane groups of
 // gram_c0 read distinct slots
 __device__ __forceinline__ int f_at(int c) { return c + 4 * (c >> 6); }
-// Channel swizzle of the fp32 row arrays (gate / Gamma, q^ fi, k^ fi, k^ fj; 132-float rows): logical channel c is
-// stored at c ^ (((c >> 5) & 3) << 2), i.e. the four 16-byte slots of the 16-channel segment of raw thread cb are
-// permuted by slot ^= cb >> 1.  The eight raw threads of a row then write 16-byte slots on distinct banks (unswizzled,
-// segments cb and cb + 4 sit 256 bytes apart and their writes conflict: 128 vs 55 cycles per wave instruction).
-__device__ __forceinline__ int swz(int c) { return c ^ (((c >> 5) & 3) << 2); }
 // hi + lo bf16 split of two fp32 values, each pair packed in one word (element 0 in the low half): hi = RNE(x),
 // lo = RNE(x - hi), one v_cvt_pk_bf16_f32 per pair
 __device__ __forceinline__ void split_bf16x2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
@@ -180,14 +174,6 @@ typedef const __attribute__((address_space(4))) float cfloat_t;
 // would wait for the next chunk's prefetched loads and for the output stores at every phase boundary; the waves of
 // this kernel exchange data through LDS alone, so completing the LDS operations (lgkmcnt(0)) is sufficient.
 
-// Sum over each group of 8 consecutive lanes (quad swaps, then the mirrored quad).
-__device__ __forceinline__ float sum8(float x) {
-    x += dpp<0xB1>(x);
-    x += dpp<0x4E>(x);
-    x += dpp<0x141>(x);
-    return x;
-}
-
 struct PfParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -216,13 +202,6 @@ struct PfParams {
                  // [R slots][H][64][128] fp16 correction operands
 };
 
-// Raw inputs of one chunk row slice: row r, channels 16 cb .. 16 cb + 15.
-struct RawRow {
-    u32x4 q[2], k[2], v[2];
-    u32x4 g[4];  // fp32 log-decay (4 x 4 floats), or bf16 raw gate in g[0..1]
-    uint32_t beta;  // fp32 bits, or the bf16 raw beta in the low half (converted when the chunk is consumed)
-};
-
 // Raw buffer descriptor over the rows [t0, t0 + L) of one token-major stream (row pitch `pitch` bytes, `bytes` bytes
 // per row used): a row past the chunk end lies outside num_records, and the buffer load returns zeros for it.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, int L, int64_t pitch, int bytes) {
@@ -231,65 +210,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, in
 }
 __device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t rs, int off) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-}
-
-// One chunk's raw row slice for this thread (row r, channels 16 cb .. 16 cb + 15); rows >= L read as zeros.  The
-// next chunk's slice is issued in three parts in three phases (q and k; v and beta; the gate): the 80 KiB a chunk
-// loads take ~1.3 k cycles of the CU's address unit, and issued at once they stall the waves that issue them.
-__device__ __forceinline__ void load_row_qk(const PfParams& p, int h, int t0, int L, int r, int cb, RawRow& x) {
-    const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
-    const int64_t qp = p.qkv_rs * 2;
-    const int qo = r * (int)qp + 32 * cb;
-    const __amdgpu_buffer_rsrc_t rq = rows_rsrc(p.q + o, L, qp, 256);
-    const __amdgpu_buffer_rsrc_t rk = rows_rsrc(p.k + o, L, qp, 256);
-    x.q[0] = bload16(rq, qo); x.q[1] = bload16(rq, qo + 16);
-    x.k[0] = bload16(rk, qo); x.k[1] = bload16(rk, qo + 16);
-}
-__device__ __forceinline__ void load_row_vb(const PfParams& p, int h, int t0, int L, int r, int cb, bool RB, RawRow& x) {
-    const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
-    const int64_t qp = p.qkv_rs * 2;
-    const int qo = r * (int)qp + 32 * cb;
-    const __amdgpu_buffer_rsrc_t rv = rows_rsrc(p.v + o, L, qp, 256);
-    x.v[0] = bload16(rv, qo); x.v[1] = bload16(rv, qo + 16);
-    const int es = RB ? 2 : 4;
-    const int64_t bp = p.beta_rs * es;
-    const __amdgpu_buffer_rsrc_t rb =
-        rows_rsrc(reinterpret_cast<const unsigned char*>(p.beta) + ((int64_t)t0 * p.beta_rs + h) * es, L, bp, es);
-    x.beta = RB ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rb, r * (int)bp, 0, 0)
-                : __builtin_amdgcn_raw_buffer_load_b32(rb, r * (int)bp, 0, 0);
-}
-template <bool RG>
-__device__ __forceinline__ void load_row_g(const PfParams& p, int h, int t0, int L, int r, int cb, RawRow& x) {
-    const int64_t go = (int64_t)t0 * p.g_rs + (int64_t)h * D;
-    if (RG) {
-        const int64_t gp = p.g_rs * 2;
-        const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const uint16_t*>(p.g) + go, L, gp, 256);
-        const int off = r * (int)gp + 32 * cb;
-        x.g[0] = bload16(rg, off); x.g[1] = bload16(rg, off + 16);
-        x.g[2] = u32x4{0u, 0u, 0u, 0u}; x.g[3] = x.g[2];
-    } else {
-        const int64_t gp = p.g_rs * 4;
-        const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const float*>(p.g) + go, L, gp, 512);
-        const int off = r * (int)gp + 64 * cb;
-        x.g[0] = bload16(rg, off); x.g[1] = bload16(rg, off + 16);
-        x.g[2] = bload16(rg, off + 32); x.g[3] = bload16(rg, off + 48);
-    }
-}
-template <bool RG>
-__device__ __forceinline__ void load_row(const PfParams& p, int h, int t0, int L, int r, int cb, bool RB, RawRow& x) {
-    load_row_qk(p, h, t0, L, r, cb, x);
-    load_row_vb(p, h, t0, L, r, cb, RB, x);
-    load_row_g<RG>(p, h, t0, L, r, cb, x);
-}
-
-__device__ __forceinline__ void unpack16(const u32x4 (&w)[2], float (&f)[16]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            f[8 * i + 2 * j] = bf2f(w[i][j] & 0xffffu);
-            f[8 * i + 2 * j + 1] = bf2f(w[i][j] >> 16);
-        }
 }
 
 // Raw inputs of one chunk for one lane.  Wave w owns the chunk's rows 8 w .. 8 w + 7; lane l of it the rows
