@@ -157,11 +157,12 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
         {
             f32x4 kfi[4], kfj[4], qfi[4];
             chunk_front<RG>(nx, w, lane, L, RB, NORM, An, p.lb, sDT, sWt, sBeta, sVt, RSV32, kfi, kfj, qfi);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(&sKA[(row0 + j) * RS32 + 4 * c4]) = kfi[j];
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int o = (row0 + j) * RS32 + 4 * c4;
-                *reinterpret_cast<f32x4*>(&sKA[o]) = kfi[j];
                 *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
                 *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
             }

@@ -139,11 +139,20 @@ __device__ __forceinline__ int gram_c0(int s, int g) { return 64 * (g & 1) + 32 
 // gram_c0 read distinct slots
 __device__ __forceinline__ int f_at(int c) { return c + 4 * (c >> 6); }
 // hi + lo bf16 split of two fp32 values, each pair packed in one word (element 0 in the low half): hi = RNE(x),
-// lo = RNE(x - hi), one v_cvt_pk_bf16_f32 per pair
+// lo = RNE(x - hi).  x - hi (exact in fp32) as a bf16 dot product with (-1, 0) or (0, -1): 4 instructions a pair
+// (v_cvt_pk_bf16_f32, two v_dot2c_f32_bf16, v_cvt_pk_bf16_f32) where widening hi and subtracting took 6; a diagonal
+// Gram wave splits 48 pairs a chunk, and its issue bounds the phase.
 __device__ __forceinline__ void split_bf16x2(float x0, float x1, uint32_t& hi, uint32_t& lo) {
     hi = f2bf2(x0, x1);
-    const float h0 = __uint_as_float(hi << 16), h1 = __uint_as_float(hi & 0xffff0000u);
-    lo = f2bf2(x0 - h0, x1 - h1);
+    const uint32_t h = hi;
+    const bf16x2_t hp = __builtin_bit_cast(bf16x2_t, h);
+    // (-1, 0) and (0, -1) from registers: as a constant this compiler encodes (-1, 0) as the inline -1.0f, which the
+    // instruction reads as (0, -1)
+    uint32_t c10, c01;
+    asm("s_mov_b32 %0, 0xbf80" : "=s"(c10));
+    asm("s_mov_b32 %0, 0xbf800000" : "=s"(c01));
+    const bf16x2_t m10 = __builtin_bit_cast(bf16x2_t, c10), m01 = __builtin_bit_cast(bf16x2_t, c01);
+    lo = f2bf2(__builtin_amdgcn_fdot2_f32_bf16(hp, m10, x0, false), __builtin_amdgcn_fdot2_f32_bf16(hp, m01, x1, false));
 }
 __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t (&w)[4]) {
     return __builtin_bit_cast(bf16x8, u32x4{w[0], w[1], w[2], w[3]});
@@ -659,15 +668,17 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             const bool pf_here = cl + 1 < nch, pf = pf_here || more;
             const int pf_h = pf_here ? h : nx_h, pf_t = pf_here ? t0 + 64 : nx_t;
             const int pf_L = pf_here ? min(64, len - 64 * (cl + 1)) : (nx_nch > 0 ? min(64, nx_len) : 0);
-            // ================= P0-P2: the wave's rows to gated operands in registers (no barrier since the walk: what
-            // this writes to LDS the walk does not read), then, once every wave has left the walk, to regions A, B, C
+            // ================= P0-P2: the wave's rows to gated operands in registers and k^ fi to region A (no barrier
+            // since the walk: the walk reads nothing that this writes), then, once every wave has left the walk, k^ fj
+            // and q^ fi to regions C and B
             f32x4 kfi[4], kfj[4], qfi[4];
             chunk_front<RG>(nx, w, lane, L, RB, NORM, An, p.lb, sDT, sWt, sBeta, sVt, RS16S, kfi, kfj, qfi);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(&sKA[(row0 + j) * RS32 + 4 * c4]) = kfi[j];
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int o = (row0 + j) * RS32 + 4 * c4;
-                *reinterpret_cast<f32x4*>(&sKA[o]) = kfi[j];
                 *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
                 *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
             }
