@@ -22,7 +22,7 @@ constexpr int RSA32 = 40;                                // -A_kk / T_II rows
 constexpr int W_HALF32 = 32 * RSW;                       // elements of a half array of W
 constexpr int C32_A = 0;                                 // k^ fi: fp32 [32][RS32]
 constexpr int C32_B = C32_A + 32 * RS32 * 4;             // q^ fi fp32 [32][RS32]; then Q~ fp16 [32][RSQ]
-constexpr int C32_BV = C32_B + 32 * RSQ * 2;             // W fp16 [2][32][RSW] (region B's upper half)
+constexpr int C32_BV = C32_B + 32 * RSQ * 2;             // -W fp16 [2][32][RSW] (region B's upper half)
 constexpr int C32_C = C32_BV + 2 * W_HALF32 * 2;         // k^ fj fp32 [32][RS32]; then Kd^T fp16 [128][RST32]
 constexpr int C32_VT = C32_C + 32 * RS32 * 4;            // V^T bf16 [128][RSV32]
 constexpr int C32_AQ = C32_VT + 128 * RSV32 * 2;         // A_qk fp16 [32][RST32] (columns permuted)
@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
     int c4 = lane & 31, row0 = 8 * w + 4 * (lane >> 5);  // the lane's channels 4 c4 .. + 3 and rows row0 .. + 3
     const float dtb = RG ? p.dt_bias[h * D + (tid & (D - 1))] : 0.f;
     const float alog = RG ? p.A_log[h] : 0.f;
-    RawRows nx;
+    RawRows<RG> nx;
     load_rows<RG>(p, h, tstart, nch > 0 ? min(32, len) : 0, row0, c4, RB, nx);  // an empty sequence loads nothing
     f32x4 S[8][2];
     {
@@ -183,7 +183,9 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                 sF[F32_Y * RSF + fc] = exp2_(t1 + (t2 + t3));
             }
         }
+        load_rows_qk(p, h, pf_t, pf_L, row0, c4, nx, 1);  // the next chunk's rows, one group a phase (see load_rows_qk)
         lds_barrier();
+        load_rows_qk(p, h, pf_t, pf_L, row0, c4, nx, 2);
         // ================= P4: Gram tiles.  Wave I (0, 1): the diagonal block's A_kk (bf16 hi + lo products of
         // k^ fi and k^ fj), then T_II = (I + L_II)^-1; wave 2 + I: the same block's A_qk (k^ fj and q^ fi), then one
         // product of block (1, 0) from fp16 operands <= 1 (reference row 15): A_kk on wave 2, A_qk on wave 3.
@@ -293,7 +295,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
         for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct) asm volatile("" : "+v"(S[dt][ct]));
-        if (pf) load_rows_qk(p, h, pf_t, pf_L, row0, c4, nx);
+        load_rows_vb(p, h, pf_t, pf_L, row0, c4, RB, nx);
         // the lane's q^ fi and k^ fj back from LDS: with 64 registers of S, holding their 32 through the Gram phase spills
         f32x4 kfj[4], qfi[4];
 #pragma unroll
@@ -323,7 +325,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             }
         }
         // ================= P6: W and U by block forward substitution (wave w: channel / value tiles 2 w, 2 w + 1)
-        if (pf) load_rows_vb(p, h, pf_t, pf_L, row0, c4, RB, nx);
+        load_rows_g<RG>(p, h, pf_t, pf_L, row0, c4, nx);
         f32x4 Ur[2][2];  // [block I][tile t]: U[token 16 I + 4 g + e][value 32 w + 16 t + m]
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -355,7 +357,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                 const f32x4 Xt = mfma16(bwh, T, z);
                 Ur[I][t] = mfma16(T, buh, z);
                 *reinterpret_cast<f16x4*>(&sW[half_at(16 * I + m, 32 * w + 8 * g + 4 * t, RSW, W_HALF32)]) =
-                    f16x4{(half_t)Xt[0], (half_t)Xt[1], (half_t)Xt[2], (half_t)Xt[3]};
+                    f16x4{(half_t)-Xt[0], (half_t)-Xt[1], (half_t)-Xt[2], (half_t)-Xt[3]};
                 if (I == 0) {
                     const f32x4 Xw = mfma16(T, bwh, z);
 #pragma unroll
@@ -365,7 +367,6 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
         }
         lds_barrier();
         // ================= P7: the walk (wave w: S[:, 32 w .. 32 w + 31])
-        if (pf) load_rows_g<RG>(p, h, pf_t, pf_L, row0, c4, nx);
         // every-n row 0: the state before the sequence's first token
         if (cl == 0 && ck_mode == 2 && every > 0 && first == 0) ck_store(ck_idx[ck_row0]);
         {
@@ -379,26 +380,21 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                         SB[s][ct][ee] = (half_t)S[2 * s][ct][ee];
                         SB[s][ct][4 + ee] = (half_t)S[2 * s + 1][ct][ee];
                     }
-            f32x4 Vp[2][2];  // W S, K step outermost
-#pragma unroll
-            for (int it = 0; it < 2; ++it)
-#pragma unroll
-                for (int ct = 0; ct < 2; ++ct) Vp[it][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 4; ++s)
 #pragma unroll
                 for (int it = 0; it < 2; ++it) {
                     const f16x8 A = *reinterpret_cast<const f16x8*>(&sW[half_at(16 * it + m, 32 * s + 8 * g, RSW, W_HALF32)]);
 #pragma unroll
-                    for (int ct = 0; ct < 2; ++ct) Vp[it][ct] = mfma32(A, SB[s][ct], Vp[it][ct]);
+                    for (int ct = 0; ct < 2; ++ct) Ur[it][ct] = mfma32(A, SB[s][ct], Ur[it][ct]);
                 }
-            f16x8 VB[2];  // V' = U - W S as fp16, tokens 4 g + e and 16 + 4 g + e
+            f16x8 VB[2];  // V' = U - W S (accumulated onto U: sW holds -W) as fp16, tokens 4 g + e and 16 + 4 g + e
 #pragma unroll
             for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
                 for (int ee = 0; ee < 4; ++ee) {
-                    VB[ct][ee] = (half_t)(Ur[0][ct][ee] - Vp[0][ct][ee]);
-                    VB[ct][4 + ee] = (half_t)(Ur[1][ct][ee] - Vp[1][ct][ee]);
+                    VB[ct][ee] = (half_t)Ur[0][ct][ee];
+                    VB[ct][4 + ee] = (half_t)Ur[1][ct][ee];
                 }
             // O^T = S^T Q~^T + V'^T A_qk^T (lane (g, m): token 16 it + m, values 32 w + 16 ct + 4 g .. + 3)
             f32x4 ao[2][2];
@@ -449,7 +445,7 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
             if (ck_mode == 1 && cs == ck_single) ck_store(ck_idx[n]);
             if (ck_mode == 2 && every > 0 && cs % every == 0 && cs < seqch) ck_store(ck_idx[ck_row0 + cs / every]);
         }
-        // no barrier here: the walk writes no LDS and reads nothing the next raw-row phase writes
+        // no barrier here: the walk writes no LDS and reads nothing the next chunk writes before its first barrier
     }
     if (pflags & PIECE_LAST) {
         if (pool) {

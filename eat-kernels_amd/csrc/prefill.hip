@@ -35,6 +35,7 @@
 #include <functional>
 #include <numeric>
 #include <queue>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -223,9 +224,10 @@ __device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t rs, int off) {
 
 // Raw inputs of one chunk for one lane.  Wave w owns the chunk's rows 8 w .. 8 w + 7; lane l of it the rows
 // row0 + j (row0 = 8 w + 4 (l / 32), j = 0 .. 3) at channels 4 (l % 32) .. + 3.
+template <bool RG>
 struct RawRows {
     u32x2 q[4], k[4], v[4];
-    u32x4 g[4];     // fp32 log-decay, or the bf16 raw gate of the 4 channels in the first two words
+    std::conditional_t<RG, u32x2, u32x4> g[4];  // the bf16 raw gate, or the fp32 log-decay, of the 4 channels
     uint32_t beta;  // row 8 w + l % 8: fp32 bits, or the bf16 raw beta in the low half (converted when consumed)
 };
 
@@ -233,22 +235,32 @@ __device__ __forceinline__ u32x2 bload8(__amdgpu_buffer_rsrc_t rs, int off) {
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
 }
 
-// One chunk's rows for this lane (row0, c4 = l % 32); rows >= L read as zeros.  The next chunk's rows are issued in
-// three parts in three phases (q and k; v and beta; the gate): the 80 KiB a chunk loads take ~1.3 k cycles of the CU's
-// address unit, and issued at once they stall the waves that issue them.
-__device__ __forceinline__ void load_rows_qk(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows& x) {
+// One chunk's rows for this lane (row0, c4 = l % 32); rows >= L read as zeros.  The next chunk's rows are issued one
+// group a phase (q beside the factors, k at the start of the Gram phase, v and beta at its end, the gate in the solve):
+// the 80 KiB a chunk loads take ~2.8 k cycles of the CU's address unit, and waves that issue them at once stand in line
+// for it.  8 x 4904 tokens, H 32: 679 us against 700 with q and k issued together at the end of the Gram phase (later
+// placements of k and the gate: 684-693).  The loads are unconditional, through descriptors of no rows when nothing
+// follows: a load under a branch keeps the old rows' 41 registers live through the whole chunk.
+template <bool RG>
+__device__ __forceinline__ void load_rows_qk(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows<RG>& x,
+                                             int parts = 3) {
     const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
     const int64_t qp = p.qkv_rs * 2;
     const int qo = row0 * (int)qp + 8 * c4;
-    const __amdgpu_buffer_rsrc_t rq = rows_rsrc(p.q + o, L, qp, 256);
-    const __amdgpu_buffer_rsrc_t rk = rows_rsrc(p.k + o, L, qp, 256);
+    if (parts & 1) {
+        const __amdgpu_buffer_rsrc_t rq = rows_rsrc(p.q + o, L, qp, 256);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x.q[j] = bload8(rq, qo + j * (int)qp);
+        for (int j = 0; j < 4; ++j) x.q[j] = bload8(rq, qo + j * (int)qp);
+    }
+    if (parts & 2) {
+        const __amdgpu_buffer_rsrc_t rk = rows_rsrc(p.k + o, L, qp, 256);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) x.k[j] = bload8(rk, qo + j * (int)qp);
+        for (int j = 0; j < 4; ++j) x.k[j] = bload8(rk, qo + j * (int)qp);
+    }
 }
+template <bool RG>
 __device__ __forceinline__ void load_rows_vb(const PfParams& p, int h, int t0, int L, int row0, int c4, bool RB,
-                                             RawRows& x) {
+                                             RawRows<RG>& x) {
     const int64_t o = (int64_t)t0 * p.qkv_rs + (int64_t)h * D;
     const int64_t qp = p.qkv_rs * 2;
     const int qo = row0 * (int)qp + 8 * c4;
@@ -264,17 +276,14 @@ __device__ __forceinline__ void load_rows_vb(const PfParams& p, int h, int t0, i
                 : __builtin_amdgcn_raw_buffer_load_b32(rb, bo, 0, 0);
 }
 template <bool RG>
-__device__ __forceinline__ void load_rows_g(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows& x) {
+__device__ __forceinline__ void load_rows_g(const PfParams& p, int h, int t0, int L, int row0, int c4, RawRows<RG>& x) {
     const int64_t go = (int64_t)t0 * p.g_rs + (int64_t)h * D;
-    if (RG) {
+    if constexpr (RG) {
         const int64_t gp = p.g_rs * 2;
         const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const uint16_t*>(p.g) + go, L, gp, 256);
         const int off = row0 * (int)gp + 8 * c4;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u32x2 y = bload8(rg, off + j * (int)gp);
-            x.g[j] = u32x4{y.x, y.y, 0u, 0u};
-        }
+        for (int j = 0; j < 4; ++j) x.g[j] = bload8(rg, off + j * (int)gp);
     } else {
         const int64_t gp = p.g_rs * 4;
         const __amdgpu_buffer_rsrc_t rg = rows_rsrc(reinterpret_cast<const float*>(p.g) + go, L, gp, 512);
@@ -284,7 +293,7 @@ __device__ __forceinline__ void load_rows_g(const PfParams& p, int h, int t0, in
     }
 }
 template <bool RG>
-__device__ __forceinline__ void load_rows(const PfParams& p, int h, int t0, int L, int row0, int c4, bool RB, RawRows& x) {
+__device__ __forceinline__ void load_rows(const PfParams& p, int h, int t0, int L, int row0, int c4, bool RB, RawRows<RG>& x) {
     load_rows_qk(p, h, t0, L, row0, c4, x);
     load_rows_vb(p, h, t0, L, row0, c4, RB, x);
     load_rows_g<RG>(p, h, t0, L, row0, c4, x);
@@ -298,7 +307,8 @@ __device__ __forceinline__ int ch_row(int k) { return 16 * (k >> 4) + ((k & 15) 
 // 32 lanes of a half wave.  Sums of squares straight from the packed bf16 pairs (v_dot2c_f32_bf16: the products are
 // exact in fp32); the halving exchange over the two 16-lane rows leaves 4 values to reduce by DPP instead of 8.
 // rsqrt(max(|x|^2, 1e-12)) through v_rsq_f32 (the IEEE sqrt is a sequence).
-__device__ __forceinline__ void row_norms(const RawRows& x, float (&rq)[4], float (&rk)[4]) {
+template <bool RG>
+__device__ __forceinline__ void row_norms(const RawRows<RG>& x, float (&rq)[4], float (&rk)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         float sq = 0.f, sk = 0.f;
@@ -330,7 +340,7 @@ __device__ __forceinline__ void row_norms(const RawRows& x, float (&rq)[4], floa
 // whose Kd^T and v accesses were two bytes wide.  Measured: 96 heads x 8,192 tokens 591 -> 566 us, 38,881 tokens x 32
 // heads 761 -> 747 us.
 template <bool RG>
-__device__ __forceinline__ void chunk_front(const RawRows& x, int w, int lane, int L, bool RB, bool NORM, float An,
+__device__ __forceinline__ void chunk_front(const RawRows<RG>& x, int w, int lane, int L, bool RB, bool NORM, float An,
                                             float lb, const float* sDT, float* sWt, float* sBeta, uint16_t* sVt,
                                             int vt_stride, f32x4 (&kfi)[4], f32x4 (&kfj)[4], f32x4 (&qfi)[4]) {
     const int c4 = lane & 31, hf = lane >> 5, row0 = 8 * w + 4 * hf;
@@ -347,7 +357,7 @@ __device__ __forceinline__ void chunk_front(const RawRows& x, int w, int lane, i
         if (lane < 8) sBeta[br] = (br >= L) ? 0.f : bx;
     }
     float d[4][4];  // [row][channel]: the clamped log-decay, then Gamma_r - Gamma_m in log2 units
-    if (RG) {
+    if constexpr (RG) {
         // g log2(e) = lb log2(e) sigmoid(e^{A_log} (x + dt_bias)), the sigmoid as 1 / (1 + 2^{An x + An dt}) (one FMA,
         // v_exp_f32, one add, v_rcp_f32), already in log2 units.  Every row is computed; rows >= L get a zero
         // multiplier (their raw gate reads as 0, so the sigmoid is finite).
@@ -487,7 +497,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     half_t* sQt = reinterpret_cast<half_t*>(lds + LDS_B);    // Q~ (channels permuted)
     float* sKB = reinterpret_cast<float*>(lds + LDS_C);      // k^ fj
     half_t* sKd = reinterpret_cast<half_t*>(lds + LDS_C);    // Kd^T (tokens permuted)
-    half_t* sW = reinterpret_cast<half_t*>(lds + LDS_BV);    // W (channels permuted), in region B's upper half
+    half_t* sW = reinterpret_cast<half_t*>(lds + LDS_BV);    // -W (channels permuted), in region B's upper half
     uint16_t* sVt = reinterpret_cast<uint16_t*>(lds + LDS_VT);  // this chunk's raw v transposed (bf16)
     half_t* sAq = reinterpret_cast<half_t*>(lds + LDS_AQ);   // A_qk (columns permuted)
     half_t* sAk = reinterpret_cast<half_t*>(lds + LDS_AK);   // -A_kk off-diagonal blocks, T_II diagonal blocks
@@ -582,7 +592,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     float dtb = RG ? p.dt_bias[cur.h * D + (tid & (D - 1))] : 0.f;
     asm volatile("" ::"s"(every), "s"(ws_arr), "s"(cur.ck_row0), "s"(cur.ck_single_raw), "s"(ck_words), "s"(cur.alog),
                  "s"(p.ws));
-    RawRows nx;
+    RawRows<RG> nx;
     // an empty sequence loads nothing
     load_rows<RG>(p, cur.h, cur.tstart, cur.nch > 0 ? min(64, cur.len) : 0, row0, c4, RB, nx);
     f32x4 S[8];
@@ -664,8 +674,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             row0 = 8 * w + 4 * (lane >> 5);
             const int t0 = tstart + 64 * cl, L = min(64, len - 64 * cl);
             // the rows fetched during this chunk: the next chunk's, or during an item's last chunk the next item's
-            // first
-            const bool pf_here = cl + 1 < nch, pf = pf_here || more;
+            // first; with neither, loads of no records: loads under a branch keep the old rows' registers (41) alive
+            // through the whole chunk for the path without them
+            const bool pf_here = cl + 1 < nch;
             const int pf_h = pf_here ? h : nx_h, pf_t = pf_here ? t0 + 64 : nx_t;
             const int pf_L = pf_here ? min(64, len - 64 * (cl + 1)) : (nx_nch > 0 ? min(64, nx_len) : 0);
             // ================= P0-P2: the wave's rows to gated operands in registers and k^ fi to region A (no barrier
@@ -714,51 +725,68 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     sF[f * RSF + f_at(c)] = exp2_(x);
                 }
             }
+            load_rows_qk(p, pf_h, pf_t, pf_L, row0, c4, nx, 1);  // the next chunk's rows, one group a phase
             lds_barrier();
-            // ================= P4: Gram tiles
+            load_rows_qk(p, pf_h, pf_t, pf_L, row0, c4, nx, 2);
+            // ================= P4: Gram tiles.  No branch inside a wave's part: the parts' LDS reads are then scheduled
+            // ahead of their use as a whole, where per-tile branches had cut them into a dozen dependent round trips
+            // (with V' accumulated onto U and the loads one group a phase: 8 x 4904 tokens, H 32, 694 -> 679 us;
+            // 8192 tokens, H 96, 562 -> 552).
             if (w < 4) {
                 const int I = w, i = 16 * I + m;
                 f32x4 akk = {0.f, 0.f, 0.f, 0.f}, aqk = akk;
+                bf16x8 Kbh[4], Kbl[4];
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     const int c0 = gram_c0(s, g);
-                    uint32_t kah[4], kal[4], qah[4], qal[4], kbh[4], kbl[4];  // bf16x8 fragments as 4 packed pairs
+                    uint32_t kah[4], kal[4], kbh[4], kbl[4];  // bf16x8 fragments as 4 packed pairs
 #pragma unroll
                     for (int hf = 0; hf < 2; ++hf) {
                         const f32x4 ka = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + c0 + 4 * hf]);
-                        const f32x4 qa = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
                         const f32x4 kb = *reinterpret_cast<const f32x4*>(&sKB[i * RS32 + c0 + 4 * hf]);
 #pragma unroll
                         for (int j = 0; j < 2; ++j) {
                             const int e = 2 * hf + j;
                             split_bf16x2(ka[2 * j], ka[2 * j + 1], kah[e], kal[e]);
-                            split_bf16x2(qa[2 * j], qa[2 * j + 1], qah[e], qal[e]);
                             split_bf16x2(kb[2 * j], kb[2 * j + 1], kbh[e], kbl[e]);
                         }
                     }
-                    const bf16x8 Kah = as_bf16x8(kah), Kal = as_bf16x8(kal), Qah = as_bf16x8(qah), Qal = as_bf16x8(qal);
-                    const bf16x8 Kbh = as_bf16x8(kbh), Kbl = as_bf16x8(kbl);
-                    akk = mfma32bf(Kah, Kbh, akk);
-                    akk = mfma32bf(Kah, Kbl, akk);
-                    akk = mfma32bf(Kal, Kbh, akk);
-                    // transposed: lane (g, m) holds row 16 I + m, columns 16 I + 4 g .. + 3
-                    aqk = mfma32bf(Kbh, Qah, aqk);
-                    aqk = mfma32bf(Kbl, Qah, aqk);
-                    aqk = mfma32bf(Kbh, Qal, aqk);
+                    const bf16x8 Kah = as_bf16x8(kah), Kal = as_bf16x8(kal);
+                    Kbh[s] = as_bf16x8(kbh);
+                    Kbl[s] = as_bf16x8(kbl);
+                    akk = mfma32bf(Kah, Kbh[s], akk);
+                    akk = mfma32bf(Kah, Kbl[s], akk);
+                    akk = mfma32bf(Kal, Kbh[s], akk);
                 }
                 f32x4 lt;
-                f16x4 aq;
                 // beta of rows 16 I + 4 g .. + 3, read whatever the mask (a read under the mask would branch and wait
                 // for every outstanding LDS operation)
                 const f32x4 bt4 = *reinterpret_cast<const f32x4*>(&sBeta[16 * I + 4 * g]);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int rr = 4 * g + e;
-                    lt[e] = (m < rr) ? bt4[e] * akk[e] : 0.f;
-                    aq[e] = (half_t)((rr <= m) ? aqk[e] : 0.f);  // A_qk[16 I + m][16 I + rr], causal within the block
-                }
-                *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * I + 4 * g), RST, AQ_HALF)]) = aq;
+                for (int e = 0; e < 4; ++e) lt[e] = (m < 4 * g + e) ? bt4[e] * akk[e] : 0.f;
                 *reinterpret_cast<f32x4*>(&sL[(I * 16 + m) * 20 + 4 * g]) = lt;
+                // A_qk's block, independent of what follows: its splits and MFMAs fill the substitution's waits
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const int c0 = gram_c0(s, g);
+                    uint32_t qah[4], qal[4];
+#pragma unroll
+                    for (int hf = 0; hf < 2; ++hf) {
+                        const f32x4 qa = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) split_bf16x2(qa[2 * j], qa[2 * j + 1], qah[2 * hf + j], qal[2 * hf + j]);
+                    }
+                    const bf16x8 Qah = as_bf16x8(qah), Qal = as_bf16x8(qal);
+                    // transposed: lane (g, m) holds row 16 I + m, columns 16 I + 4 g .. + 3
+                    aqk = mfma32bf(Kbh[s], Qah, aqk);
+                    aqk = mfma32bf(Kbl[s], Qah, aqk);
+                    aqk = mfma32bf(Kbh[s], Qal, aqk);
+                }
+                f16x4 aq;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)  // A_qk[16 I + m][16 I + 4 g + e], causal within the block
+                    aq[e] = (half_t)((4 * g + e <= m) ? aqk[e] : 0.f);
+                *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * I + 4 * g), RST, AQ_HALF)]) = aq;
                 // T_II = (I + L_II)^-1 of this wave's block while waves 4..7 still work on the off-diagonal blocks:
                 // lane j (every group of 16 lanes computes the same columns; lanes 0..15 write) solves column j by
                 // right-looking substitution.  The wave reads back the block it has just written: a wave's LDS
@@ -773,8 +801,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         float col[16];
 #pragma unroll
                         for (int q4 = 0; q4 < 4; ++q4) {
-                            const f32x4 c4 = *reinterpret_cast<const f32x4*>(&Lb[k * 20 + 4 * q4]);
-                            col[4 * q4] = c4[0]; col[4 * q4 + 1] = c4[1]; col[4 * q4 + 2] = c4[2]; col[4 * q4 + 3] = c4[3];
+                            const f32x4 c4v = *reinterpret_cast<const f32x4*>(&Lb[k * 20 + 4 * q4]);
+                            col[4 * q4] = c4v[0]; col[4 * q4 + 1] = c4v[1]; col[4 * q4 + 2] = c4v[2]; col[4 * q4 + 3] = c4v[3];
                         }
 #pragma unroll
                         for (int ii = k + 1; ii < 16; ++ii) x[ii] -= col[ii] * x[k];
@@ -790,38 +818,37 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     }
                 }
             } else {
-                const int I = (w == 4) ? 1 : ((w == 5) ? 2 : 3);
-                const int J0 = (w == 7) ? 2 : 0;
-                const int nJ = (w == 4 || w == 7) ? 1 : 2;
-                const int i = 16 * I + m;
-                f32x4 akk[2], aqk[2];
+                // block row I, NJ column blocks from J0 (compile-time: one straight-line copy per wave)
+                auto off_diagonal = [&](auto Ic, auto J0c, auto NJc) {
+                    constexpr int I = decltype(Ic)::value, J0 = decltype(J0c)::value, NJ = decltype(NJc)::value;
+                    const int i = 16 * I + m;
+                    f32x4 akk[NJ], aqk[NJ];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) { akk[t] = f32x4{0.f, 0.f, 0.f, 0.f}; aqk[t] = akk[t]; }
+                    for (int t = 0; t < NJ; ++t) { akk[t] = f32x4{0.f, 0.f, 0.f, 0.f}; aqk[t] = akk[t]; }
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int c0 = gram_c0(s, g);
-                    f16x8 ka, qa;
+                    for (int s = 0; s < 4; ++s) {
+                        const int c0 = gram_c0(s, g), f0 = f_at(c0);
+                        f16x8 ka, qa;
 #pragma unroll
-                    for (int hf = 0; hf < 2; ++hf) {
-                        const f32x4 a = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + c0 + 4 * hf]);
-                        const f32x4 q4 = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
-                        const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[(F_A + I - 1) * RSF + f_at(c0) + 4 * hf]);
+                        for (int hf = 0; hf < 2; ++hf) {
+                            const f32x4 a = *reinterpret_cast<const f32x4*>(&sKA[i * RS32 + c0 + 4 * hf]);
+                            const f32x4 q4 = *reinterpret_cast<const f32x4*>(&sQA[i * RS32 + c0 + 4 * hf]);
+                            const f32x4 fa = *reinterpret_cast<const f32x4*>(&sF[(F_A + I - 1) * RSF + f0 + 4 * hf]);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            ka[4 * hf + j] = (half_t)(a[j] * fa[j]);
-                            qa[4 * hf + j] = (half_t)(q4[j] * fa[j]);
+                            for (int j = 0; j < 4; ++j) {
+                                ka[4 * hf + j] = (half_t)(a[j] * fa[j]);
+                                qa[4 * hf + j] = (half_t)(q4[j] * fa[j]);
+                            }
                         }
-                    }
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        if (t < nJ) {
-                            const int J = J0 + t, jr = 16 * J + m;
-                            const int fb = F_B + (I * (I - 1)) / 2 + J;
+                        for (int t = 0; t < NJ; ++t) {
+                            const int jr = 16 * (J0 + t) + m;
+                            constexpr int fb0 = F_B + (I * (I - 1)) / 2 + J0;
                             f16x8 kb;
 #pragma unroll
                             for (int hf = 0; hf < 2; ++hf) {
                                 const f32x4 b = *reinterpret_cast<const f32x4*>(&sKB[jr * RS32 + c0 + 4 * hf]);
-                                const f32x4 fbv = *reinterpret_cast<const f32x4*>(&sF[fb * RSF + f_at(c0) + 4 * hf]);
+                                const f32x4 fbv = *reinterpret_cast<const f32x4*>(&sF[(fb0 + t) * RSF + f0 + 4 * hf]);
 #pragma unroll
                                 for (int j = 0; j < 4; ++j) kb[4 * hf + j] = (half_t)(b[j] * fbv[j]);
                             }
@@ -829,11 +856,9 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                             aqk[t] = mfma32(kb, qa, aqk[t]);  // columns 16 J + 4 g .. + 3
                         }
                     }
-                }
-                const float nb = -sBeta[i];
+                    const float nb = -sBeta[i];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (t < nJ) {
+                    for (int t = 0; t < NJ; ++t) {
                         const int J = J0 + t;
                         f16x4 ak, al, aq;
 #pragma unroll
@@ -848,7 +873,16 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         if (PREC) *reinterpret_cast<f16x4*>(&sAk[(16 * J + m) * RS16S + 16 * I + 4 * g]) = al;
                         *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * J + 4 * g), RST, AQ_HALF)]) = aq;
                     }
-                }
+                };
+                using std::integral_constant;
+                if (w == 4)
+                    off_diagonal(integral_constant<int, 1>{}, integral_constant<int, 0>{}, integral_constant<int, 1>{});
+                else if (w == 5)
+                    off_diagonal(integral_constant<int, 2>{}, integral_constant<int, 0>{}, integral_constant<int, 2>{});
+                else if (w == 6)
+                    off_diagonal(integral_constant<int, 3>{}, integral_constant<int, 0>{}, integral_constant<int, 2>{});
+                else
+                    off_diagonal(integral_constant<int, 3>{}, integral_constant<int, 2>{}, integral_constant<int, 1>{});
             }
             // The initial state loads (issued in the prologue or at the item's start) complete here, before any
             // next-chunk row is in flight: an empty use of S makes the compiler's wait for them fall at this point,
@@ -856,11 +890,10 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             // walk, where it would also wait for the prefetched rows.
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) asm volatile("" : "+v"(S[dt]));
-            // the next chunk's q, k rows: issued here, consumed at the next P0 (their registers are free during P1..P4)
-            if (pf) load_rows_qk(p, pf_h, pf_t, pf_L, row0, c4, nx);
+            load_rows_vb(p, pf_h, pf_t, pf_L, row0, c4, RB, nx);
             lds_barrier();  // regions B and C are rewritten below
             {
-                // the lane still holds its rows' q^ fi and k^ fj; its block is I = w / 2
+                // the lane's block is I = w / 2
                 const f32x4 xf = *reinterpret_cast<const f32x4*>(&sF[(F_X + (w >> 1)) * RSF + f_at(4 * c4)]);
                 const f32x4 yf = *reinterpret_cast<const f32x4*>(&sF[(F_Y + (w >> 1)) * RSF + f_at(4 * c4)]);
                 const int qc = 32 * (c4 >> 3) + 8 * (c4 & 3) + (c4 & 4);  // stored position of channel 4 c4
@@ -885,7 +918,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             // operand reads before the layouts) passed the barrier above.  The walk reads the layouts after the solve's
             // barrier.
             // ================= P6: W and U by block forward substitution (wave w: channel / value tile w)
-            if (pf) load_rows_vb(p, pf_h, pf_t, pf_L, row0, c4, RB, nx);
+            load_rows_g<RG>(p, pf_h, pf_t, pf_L, row0, c4, nx);
             f32x4 Ur[4];
             {
                 const int c = 16 * w + m;
@@ -940,7 +973,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         Ur[I] = mfma16(Tl, buh, mfma16(T, bul, Ur[I]));
                     }
                     *reinterpret_cast<f16x4*>(&sW[half_at(16 * I + m, 32 * (w >> 1) + 8 * g + 4 * (w & 1), RSW, W_HALF)]) =
-                        f16x4{(half_t)Xt[0], (half_t)Xt[1], (half_t)Xt[2], (half_t)Xt[3]};
+                        f16x4{(half_t)-Xt[0], (half_t)-Xt[1], (half_t)-Xt[2], (half_t)-Xt[3]};
                     if (I < 3) {
                         split4(Xw[I], Xh[I], Xl[I]);
                         split4(Ur[I], Uh[I], Ul[I]);
@@ -952,7 +985,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             if (RG && !pf_here && more && tid < D) sDT[tid] = dtb_next;
             lds_barrier();
             // ================= P7: the walk
-            if (pf) load_rows_g<RG>(p, pf_h, pf_t, pf_L, row0, c4, nx);
             // every-n row 0 is the state before the sequence's first token: stored before the first walk changes S
             // (here rather than in the prologue, so that nothing before the first walk waits for the state loads)
             if (cl == 0 && ck_mode == 2 && every > 0 && first == 0) ck_store(ck_idx[ck_row0]);
@@ -967,9 +999,11 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         PB[s][e] = (half_t)Pm[2 * s][e];
                         PB[s][4 + e] = (half_t)Pm[2 * s + 1][e];
                     }
-                f32x4 Vp[4], Wp[4];  // W S and W P, K step outermost (eight independent MFMA chains per step)
+                // V' = U - W S accumulated onto U, and -W P, K step outermost (eight independent MFMA chains per step)
+                f32x4 (&Vp)[4] = Ur;
+                f32x4 Wp[4];
 #pragma unroll
-                for (int it = 0; it < 4; ++it) { Vp[it] = f32x4{0.f, 0.f, 0.f, 0.f}; Wp[it] = Vp[it]; }
+                for (int it = 0; it < 4; ++it) Wp[it] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -978,10 +1012,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         Vp[it] = mfma32(A, SB[s], Vp[it]);
                         Wp[it] = mfma32(A, PB[s], Wp[it]);
                     }
-#pragma unroll
-                for (int it = 0; it < 4; ++it)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) { Vp[it][e] = Ur[it][e] - Vp[it][e]; Wp[it][e] = -Wp[it][e]; }
                 f16x8 VB[2], WB[2], VL[2], WL[2];  // V' and -W P; PREC: also their low parts (fp16 pairs)
 #pragma unroll
                 for (int s = 0; s < 2; ++s)
@@ -1049,21 +1079,15 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         SB[s][e] = (half_t)S[2 * s][e];
                         SB[s][4 + e] = (half_t)S[2 * s + 1][e];
                     }
-                f32x4 Vp[4];
-                // W S with the K step outermost: the four token tiles' MFMAs of one step are independent, so none
-                // waits for the previous one's accumulator
-#pragma unroll
-                for (int it = 0; it < 4; ++it) Vp[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+                // V' = U - W S accumulated onto U, with the K step outermost: the four token tiles' MFMAs of one step
+                // are independent, so none waits for the previous one's accumulator
+                f32x4 (&Vp)[4] = Ur;
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
 #pragma unroll
                     for (int it = 0; it < 4; ++it)
                         Vp[it] = mfma32(*reinterpret_cast<const f16x8*>(&sW[half_at(16 * it + m, 32 * s + 8 * g, RSW, W_HALF)]), SB[s],
                                         Vp[it]);
-#pragma unroll
-                for (int it = 0; it < 4; ++it)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) Vp[it][e] = Ur[it][e] - Vp[it][e];
                 f16x8 VB[2], VL[2];  // V'; PREC: also its low part (an fp16 pair)
 #pragma unroll
                 for (int s = 0; s < 2; ++s)
@@ -1131,8 +1155,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 if (ck_mode == 2 && every > 0 && cs % every == 0 && cs < seqch) ck_store(ck_idx[ck_row0 + cs / every]);
             }
             // no barrier here: the walk writes no LDS (its outputs go straight to `out`) and reads none of what the
-            // next chunk's raw-row phase writes (raw v rows, gate rows, beta); the barrier after that phase orders
-            // everything the walk reads before the cumsum and factors overwrite it
+            // next chunk writes before its first barrier (k^ fi, raw v, gate totals, beta); that barrier orders
+            // everything the walk reads before the factors and operands overwrite it
         }
         if (fix) {  // the piece's local end state (blocked order) and transition (fp16) for the scan; LDS is free now
             float* st0 = reinterpret_cast<float*>(lds);
