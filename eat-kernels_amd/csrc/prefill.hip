@@ -687,12 +687,6 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
 #pragma unroll
             for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(&sKA[(row0 + j) * RS32 + 4 * c4]) = kfi[j];
             lds_barrier();
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int o = (row0 + j) * RS32 + 4 * c4;
-                *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
-                *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
-            }
             {
                 // block factors, one thread per channel and factor group; qd is wave-uniform (128 threads per value):
                 // the row selection below branches on the scalar unit
@@ -724,6 +718,14 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     }
                     sF[f * RSF + f_at(c)] = exp2_(x);
                 }
+            }
+            // after the factors, whose reads of the gate totals would otherwise queue behind 64 KiB of writes in the LDS
+            // (8 x 4904 tokens, H 32: 654 -> 645 us)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int o = (row0 + j) * RS32 + 4 * c4;
+                *reinterpret_cast<f32x4*>(&sKB[o]) = kfj[j];
+                *reinterpret_cast<f32x4*>(&sQA[o]) = qfi[j];
             }
             load_rows_qk(p, pf_h, pf_t, pf_L, row0, c4, nx, 1);  // the next chunk's rows, one group a phase
             lds_barrier();
@@ -917,6 +919,13 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
             // none of which the layouts above write; it writes W into region B's upper half, whose last reader (the
             // operand reads before the layouts) passed the barrier above.  The walk reads the layouts after the solve's
             // barrier.
+            // The two waves of a SIMD are w and w + 4, and at equal priority the older one (w < 4) wins every issue: it
+            // ran ahead through the solve and the walk and into the next chunk's front, then waited there ~2.1 k of its
+            // 17 k cycles while the other finished alone, at a lone wave's half issue rate.  The younger half first from
+            // here to the walk's end, the older half (by age) in the front: both reach the next barrier together
+            // (8 x 4904 tokens, H 32: 668 -> 645 us; 8192 tokens, H 96: 552 -> 538; the walk alone, the front alone or
+            // a switch inside the walk 648-664 us, the Gram phase or the factors included 657-679).
+            if (w >= 4) __builtin_amdgcn_s_setprio(1);
             // ================= P6: W and U by block forward substitution (wave w: channel / value tile w)
             load_rows_g<RG>(p, pf_h, pf_t, pf_L, row0, c4, nx);
             f32x4 Ur[4];
@@ -1139,6 +1148,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     }
                 }
             }
+            if (w >= 4) __builtin_amdgcn_s_setprio(0);
             // checkpoints at chunk boundaries, counted in chunks of the whole sequence
             const int cs = first + cl + 1;
             if (fix) {  // the pair (S_loc, P) of this chunk boundary; the row is composed once S_start is known
