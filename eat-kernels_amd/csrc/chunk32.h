@@ -224,27 +224,11 @@ __global__ void __launch_bounds__(C32_THREADS) __attribute__((amdgpu_waves_per_e
                 f32x4 lt;
                 const f32x4 bt4 = *reinterpret_cast<const f32x4*>(&sBeta[16 * I + 4 * g]);
 #pragma unroll
-                for (int ee = 0; ee < 4; ++ee) lt[ee] = (m < 4 * g + ee) ? bt4[ee] * acc[ee] : 0.f;
+                for (int ee = 0; ee < 4; ++ee) lt[ee] = (m < 4 * g + ee) ? -(bt4[ee] * acc[ee]) : 0.f;
                 *reinterpret_cast<f32x4*>(&sL[(I * 16 + m) * 20 + 4 * g]) = lt;
-                const float* Lb = sL + I * 16 * 20;  // column k of L_II is the contiguous row k; the wave reads back
-                float x[16];                         // what it has just written (its LDS operations complete in order)
+                const f32x4 x = invert_unit_lower(sL + I * 16 * 20, g, m);
 #pragma unroll
-                for (int ii = 0; ii < 16; ++ii) x[ii] = (ii == m) ? 1.f : 0.f;
-#pragma unroll
-                for (int k = 0; k < 15; ++k) {
-                    float col[16];
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4) {
-                        const f32x4 c4 = *reinterpret_cast<const f32x4*>(&Lb[k * 20 + 4 * q4]);
-                        col[4 * q4] = c4[0]; col[4 * q4 + 1] = c4[1]; col[4 * q4 + 2] = c4[2]; col[4 * q4 + 3] = c4[3];
-                    }
-#pragma unroll
-                    for (int ii = k + 1; ii < 16; ++ii) x[ii] -= col[ii] * x[k];
-                }
-                if (g == 0) {
-#pragma unroll
-                    for (int ii = 0; ii < 16; ++ii) sAk[(16 * I + ii) * RSA32 + 16 * I + m] = (half_t)x[ii];
-                }
+                for (int ee = 0; ee < 4; ++ee) sAk[(16 * I + 4 * g + ee) * RSA32 + 16 * I + m] = (half_t)x[ee];
             } else {
                 f16x4 aq;
 #pragma unroll

@@ -341,6 +341,34 @@ def test_row_group_edges(oracle, raw, cus, chunk64):
         assert rel_frob(f32(fin[n]), rf[n]) <= STATE_TOL, f"seq {n} (len {lens[n]})"
 
 
+@pytest.mark.parametrize("form", ["whole", "precise", "lists", "chunk32"])
+def test_correlated_keys(oracle, form):
+    """Keys with a common direction (cosines ~0.5), beta ~0.9 and hardly any decay: the 16 x 16 systems I + L of the
+    solve are far from the identity (entries ~0.45 everywhere below the diagonal), so every block and row of their
+    inverses counts; lengths end inside and at the edges of the 4-row blocks.  Bars as in the other parity tests."""
+    kda = _kda()
+    H, lens = 2, [1, 4, 5, 15, 16, 17, 31, 33, 50, 64, 77, 200]
+    _say(f"correlated keys, {form}")
+    g = gen(142)
+    T = sum(lens)
+    q = torch.randn(T, H, D, generator=g).bfloat16()
+    k = (torch.randn(T, H, D, generator=g) + torch.randn(1, H, D, generator=g)).bfloat16()
+    v = torch.randn(T, H, D, generator=g).bfloat16()
+    gl = -1e-3 * torch.rand(T, H, D, generator=g)
+    bt = 0.85 + 0.1 * torch.rand(T, H, generator=g)
+    h0 = torch.randn(len(lens), H, D, D, generator=g) * 0.05
+    cus = None if form in ("whole", "precise") else 4
+    meta = _list_meta(kda, lens, H, cus, form != "chunk32") if cus else None
+    o, fin = kda.chunk_kda(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), gl[None].to(DEV), bt[None].to(DEV),
+                           initial_state=h0.to(DEV), output_final_state=True, cu_seqlens=torch.tensor(_cu(lens)).to(DEV),
+                           precise=form == "precise", meta=meta)
+    torch.cuda.synchronize()
+    ro, rf = oracle.prefill_plain(f32(q), f32(k), f32(v), f32(gl), f32(bt), _cu(lens), initial_state=f32(h0), precision=64)
+    _check_out(o[0], ro, "correlated keys", _cu(lens))
+    for n in range(len(lens)):
+        assert rel_frob(f32(fin[n]), rf[n]) <= STATE_TOL, f"seq {n} (len {lens[n]})"
+
+
 def _pages(slots, H, taps, g):
     """vLLM hybrid page layout (kda/mi350x/CONTRACT.md:60-67): conv state then SSM state per padded page."""
     dim = H * D
