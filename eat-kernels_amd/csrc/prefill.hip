@@ -1506,18 +1506,20 @@ __device__ __forceinline__ void ck_body(const PfParams& p, const int32_t* __rest
 
 // The outputs of later pieces: O = partial (fp16, as the chunk kernel left it in `out`) + scale R S_start, stored as
 // bf16.  One workgroup of 256 threads (4 waves) per (group of up to FX_GROUP chunks of one piece, head): the start
-// state goes to LDS once per group (fp16 [v][k], rows of 17 16-byte slots, slot s of row v stored at s ^ 4 (v / 32)
-// so that the A-fragment reads below hit 16 distinct slots).  Wave w takes tokens 16 w .. 16 w + 15 of every chunk:
-// 16x16x32 f16 MFMAs with the state as the A operand (tile vt, A row i <-> value 32 (i / 4) + 4 vt + i % 4) and the R
-// rows as the B operand, so lane (g, m) ends with the 32 consecutive values 32 g .. 32 g + 31 of token 16 w + m (four
+// state goes to LDS once per group (fp16 [v][k], 16 slots of 16 bytes a row, slot s of row v stored at s ^ h(v) with
+// h(v) = 4 (v / 8 % 4) + v % 4, a bijection over the 16 rows an A fragment reads: its reads hit 16 distinct slots).
+// Wave w takes tokens 16 w .. 16 w + 15 of every chunk: 16x16x32 f16 MFMAs with the state as the A operand (tile vt,
+// A row i <-> value 32 (vt / 2) + 8 (i / 4) + 4 (vt % 2) + i % 4) and the R
+// rows as the B operand, so lane (g, m) ends with the values 32 i + 8 g .. + 7 (i = 0 .. 3) of token 16 w + m, and
+// the four lanes of a token load and store 64 contiguous bytes at a time (four
 // 16-byte loads of the partial and four stores).  Each chunk's R rows and partials are loaded one chunk ahead, through
 // buffer descriptors that end at the group's last token and last R tile: rows past them read zeros and their stores
 // are dropped, so no access sits under a branch.
 constexpr int FX_THREADS = 256;
 constexpr int FX_GROUP = 2;  // measured: 2 chunks per group beats 1, 4 and 8 (start-state reads vs. tail)
-constexpr int FX_ROW = 17 * 16;        // bytes per fp16 state row in LDS
+constexpr int FX_ROW = 16 * 16;        // bytes per fp16 state row in LDS
 constexpr int FX_SMEM = D * FX_ROW;
-__device__ __forceinline__ int fx_slot(int v, int s) { return v * FX_ROW + 16 * (s ^ (4 * (v >> 5))); }
+__device__ __forceinline__ int fx_slot(int v, int s) { return v * FX_ROW + 16 * (s ^ (((v >> 1) & 12) | (v & 3))); }
 __device__ __forceinline__ void fixup_body(const PfParams& p, const int32_t* __restrict__ tab, unsigned char* lds,
                                            int blk) {
     const int H = p.H;
@@ -1541,8 +1543,8 @@ __device__ __forceinline__ void fixup_body(const PfParams& p, const int32_t* __r
     const int nchk = (L + 63) >> 6;
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t*>(R0), (short)0, (int)((nchk - 1) * rstep * 2 + 64 * D * 2), 0x00020000);
-    const int roff = (tok * D + 8 * g) * 2, col = 64 * g;
-    // one chunk's operands of this lane: R row tok (k = 32 ks + 8 g .. + 7) and the partial values 32 g .. + 31
+    const int roff = (tok * D + 8 * g) * 2, col = 16 * g;
+    // one chunk's operands of this lane: R row tok (k = 32 ks + 8 g .. + 7) and the partial values 32 i + 8 g .. + 7
     struct Ops { f16x8 X[4]; f16x8 part[4]; };
     auto load = [&](Ops& b, int c0) {
         const int rbase = (int)((c0 >> 6) * rstep * 2) + roff;
@@ -1550,7 +1552,7 @@ __device__ __forceinline__ void fixup_body(const PfParams& p, const int32_t* __r
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             b.X[i] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rb, rbase + 64 * i, 0, 0));
-            b.part[i] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(ob, obase + 16 * i, 0, 0));
+            b.part[i] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(ob, obase + 64 * i, 0, 0));
         }
     };
     // wait for b's loads here (later loads stay in flight) and keep the next chunk's loads above this point
@@ -1566,14 +1568,14 @@ __device__ __forceinline__ void fixup_body(const PfParams& p, const int32_t* __r
 #pragma unroll
         for (int vt = 0; vt < 8; ++vt) {
             acc[vt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const int v = 32 * (m >> 2) + 4 * vt + (m & 3);
+            const int v = 32 * (vt >> 1) + 8 * (m >> 2) + 4 * (vt & 1) + (m & 3);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks)
                 acc[vt] = mfma32(*reinterpret_cast<const f16x8*>(lds + fx_slot(v, 4 * ks + g)), b.X[ks], acc[vt]);
         }
         const int obase = (c0 + tok) * rs + col;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {  // values 32 g + 8 i .. + 7 = tiles 2 i and 2 i + 1
+        for (int i = 0; i < 4; ++i) {  // values 32 i + 8 g .. + 7 = tiles 2 i and 2 i + 1
             const f16x8& pt = b.part[i];
             const f32x4& a0 = acc[2 * i];
             const f32x4& a1 = acc[2 * i + 1];
@@ -1582,7 +1584,7 @@ __device__ __forceinline__ void fixup_body(const PfParams& p, const int32_t* __r
             r.y = f2bf((float)pt[2] + p.scale * a0[2]) | (f2bf((float)pt[3] + p.scale * a0[3]) << 16);
             r.z = f2bf((float)pt[4] + p.scale * a1[0]) | (f2bf((float)pt[5] + p.scale * a1[1]) << 16);
             r.w = f2bf((float)pt[6] + p.scale * a1[2]) | (f2bf((float)pt[7] + p.scale * a1[3]) << 16);
-            __builtin_amdgcn_raw_buffer_store_b128(r, ob, obase + 16 * i, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(r, ob, obase + 64 * i, 0, 0);
         }
     };
     // each chunk's loads are issued one chunk ahead; the loop is unrolled whole (straight-line waits).  The first
