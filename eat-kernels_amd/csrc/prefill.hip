@@ -218,8 +218,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, in
     const int num = L > 0 ? (int)((int64_t)(L - 1) * pitch + bytes) : 0;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, num, 0x00020000);
 }
+// The rows are read once: non-temporal, so that they displace less of what the passes read again (outputs and R of
+// split sequences, start states).  12 sequences / 16 k tokens, H 12: 155.6 -> 153 us; 8 x 4904, H 32: 640 -> 635; equal
+// elsewhere.  (The fixup's own loads or stores non-temporal: 1-2 % slower, they do hit.)
+constexpr int AUX_NT = 2;
 __device__ __forceinline__ u32x4 bload16(__amdgpu_buffer_rsrc_t rs, int off) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, AUX_NT));
 }
 
 // Raw inputs of one chunk for one lane.  Wave w owns the chunk's rows 8 w .. 8 w + 7; lane l of it the rows
@@ -232,7 +236,7 @@ struct RawRows {
 };
 
 __device__ __forceinline__ u32x2 bload8(__amdgpu_buffer_rsrc_t rs, int off) {
-    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, AUX_NT));
 }
 
 // One chunk's rows for this lane (row0, c4 = l % 32); rows >= L read as zeros.  The next chunk's rows are issued one
