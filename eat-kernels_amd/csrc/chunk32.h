@@ -1,7 +1,7 @@
 // The chunk walk on 32-token chunks with a 4-wave workgroup (included by prefill.hip, inside its namespace).
 //
-// chunk_kernel keeps a 64-token chunk's operands in 156 KiB of LDS, so a CU holds one workgroup: its 8 waves (two
-// per SIMD) meet at the same five barriers per chunk and stall together.  Here a chunk is 32 tokens, the row arrays
+// chunk_kernel keeps a 64-token chunk's operands in 158 KiB of LDS, so a CU holds one workgroup: its 8 waves (two
+// per SIMD) meet at the same four barriers per chunk and stall together.  Here a chunk is 32 tokens, the row arrays
 // halve and the workgroup needs 72 KiB, so two independent workgroups share a CU: still two waves per SIMD, but from
 // workgroups whose barriers and dependent chains do not line up.  Per token the work is the same (the Gram and solve
 // blocks shrink with the chunk; the per-chunk state work -- decay, fp16 copies of S -- doubles).  Each wave keeps a
@@ -10,8 +10,9 @@
 // model has it finish first, and launches in the precise mode keep chunk_kernel.
 //
 // Same algorithm, phases and operand conventions as chunk_kernel, with two row blocks of 16 instead of four:
-//   P0-P2 rows to gated operands in registers (chunk_front), then the 7 block-factor rows, P4 Gram tiles (wave I = 0 / 1: diagonal block I's A_kk with the bf16 hi / lo split, then T_II;
-//   wave 2 + I: its A_qk, then one product of block (1, 0)), P5 Q~ and Kd^T layouts (tokens permuted by pos32),
+//   P0-P2 rows to gated operands in registers (chunk_front), then the 7 block-factor rows, P4 Gram tiles (wave I = 0
+//   / 1: diagonal block I's A_kk with the bf16 hi / lo split, then T_II; wave 2 + I: its A_qk, then one product of
+//   block (1, 0)), P5 Q~ and Kd^T layouts (tokens permuted by pos32),
 //   P6 W / U (wave w: channel / value tiles 2 w, 2 w + 1),
 //   P7 the walk (wave w: S[:, 32 w .. 32 w + 31], K step outermost).  Checkpoints fall on 64-token boundaries, i.e.
 //   after every second chunk (or after the last chunk of the sequence).
@@ -31,7 +32,7 @@ constexpr int C32_F = C32_AK + 32 * RSA32 * 2;           // factor rows [7][RSF]
 constexpr int C32_WT = C32_F + 7 * RSF * 4;              // gate totals of the 4 waves' rows [4][128] fp32
 constexpr int C32_BETA = C32_WT + 4 * 128 * 4;           // [32] fp32
 constexpr int C32_DT = C32_BETA + 32 * 4;                // An dt_bias [128] fp32 (gate in the kernel)
-constexpr int C32_L = C32_DT + 128 * 4;                  // A_kk diagonal blocks, column-major [2][16][20] fp32
+constexpr int C32_L = C32_DT + 128 * 4;                  // -L_II diagonal blocks, column-major [2][16][20] fp32
 constexpr int C32_TOTAL = C32_L + 2 * 16 * 20 * 4;
 static_assert(32 * RS32 * 4 <= 32 * RSQ * 2 + 2 * W_HALF32 * 2, "q^ fi fits region B");
 static_assert(128 * RST32 * 2 <= 32 * RS32 * 4, "Kd^T fits region C");

@@ -19,7 +19,7 @@
 //   P4  Gram tiles on MFMA: the four diagonal 16 x 16 blocks from bf16 hi + lo operands (3 MFMAs: hi.hi + hi.lo +
 //       lo.hi; their gated operands span e^{+-8|g|}), the six off-diagonal blocks from fp16 operands <= 1 (the
 //       reference point is the last row before the row block); each diagonal wave then inverts its block,
-//       (I + L_II)^-1 by forward substitution in fp32, while the off-diagonal waves finish
+//       (I + L_II)^-1 by forward substitution in fp32 by 4-row blocks, while the off-diagonal waves finish
 //   P5  Q e^Gamma and K e^{Gamma_c - Gamma} (from the lane's registers) to LDS in the walk's operand layouts
 //   P6  W and U by block forward substitution on MFMA: X_I = T_II (B_I - sum_{J<I} A_IJ X_J); wave w owns key
 //       channels [16w, 16w+16) of W and value columns [16w, 16w+16) of U, so no wave waits for another
@@ -79,7 +79,7 @@ constexpr int LDS_F = LDS_AK + 64 * RS16S * 2;
 constexpr int LDS_WT = LDS_F + 18 * RSF * 4;    // gate totals of the 8 waves' rows [8][128]; PREC: then T_II's low parts
 constexpr int LDS_BETA = LDS_WT + 8 * 128 * 4;
 constexpr int LDS_DT = LDS_BETA + 64 * 4;       // An dt_bias of the head (gate-in-kernel) fp32 [128]
-constexpr int LDS_L = LDS_DT + 128 * 4;         // A_kk diagonal blocks, transposed: [block][column][row], rows padded to 20
+constexpr int LDS_L = LDS_DT + 128 * 4;         // -L_II diagonal blocks, transposed: [block][column][row], rows padded to 20
 constexpr int LDS_TOTAL = LDS_L + 4 * 16 * 20 * 4;
 static_assert(LDS_TOTAL <= 160 * 1024, "one workgroup per CU");
 static_assert(W_HALF * 2 % 256 == 0 && AQ_HALF * 2 % 256 == 0 && KD_HALF * 2 % 256 == 0, "half arrays share their banks");
