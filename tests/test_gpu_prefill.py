@@ -43,11 +43,29 @@ def _list_meta(kda, lens, H, cus, chunk64=True, **kw):
     return meta
 
 
+def _form_meta(kda, lens, H, form, **kw):
+    """A plan that runs one form of the chunk kernel: "split" (long sequences cut into pieces, for 256 CUs), "whole" (one
+    workgroup per uncut sequence and head, for the first CU count that plans so), "lists" and "chunk32" (_list_meta for
+    4 CUs)."""
+    if form in ("lists", "chunk32"):
+        return _list_meta(kda, lens, H, 4, form == "lists", **kw)
+    if form == "split":
+        meta = kda.plan(torch.tensor(_cu(lens)), H, device=DEV, num_cus=256, **kw)
+        assert meta.split != (0, 0), meta.split
+        return meta
+    assert form == "whole"
+    for cus in range(1, 257):
+        meta = kda.plan(torch.tensor(_cu(lens)), H, num_cus=cus, **kw)
+        if meta.split == (0, 0) and int(meta.plan.chunk_grid) == 0 and int(meta.plan.chunk32) == 0:
+            return kda.plan(torch.tensor(_cu(lens)), H, device=DEV, num_cus=cus, **kw)
+    raise AssertionError(f"no CU count plans {lens} x {H} as one workgroup per whole sequence")
+
+
 def _plain_case(oracle, H, lens, seed, init=True, gscale=1.0, heads_checked=None, gmod=None, precise=False, cus=None,
-                chunk64=True):
+                chunk64=True, form=None):
     kda = _kda()
     _say(f"plain H={H} lens={lens[:10]} init={init} seed={seed}" + (" precise" if precise else "") +
-         (f" {'lists' if chunk64 else '32-token kernel'} on {cus} CUs" if cus else ""))
+         (f" {'lists' if chunk64 else '32-token kernel'} on {cus} CUs" if cus else "") + (f" {form}" if form else ""))
     g = gen(seed)
     T = int(sum(lens))
     q, k, v, gg, beta = config_inputs(T, H, g)
@@ -57,7 +75,7 @@ def _plain_case(oracle, H, lens, seed, init=True, gscale=1.0, heads_checked=None
     N = len(lens)
     h0 = torch.randn(N, H, D, D, generator=g) * 0.02 if init else None
     cu = torch.tensor(_cu(lens), dtype=torch.int32)
-    meta = _list_meta(kda, lens, H, cus, chunk64) if cus else None
+    meta = _form_meta(kda, lens, H, form) if form else _list_meta(kda, lens, H, cus, chunk64) if cus else None
     o, fin = kda.chunk_kda(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), gg[None].to(DEV), beta[None].to(DEV),
                            initial_state=h0.to(DEV) if init else None, output_final_state=True, cu_seqlens=cu.to(DEV),
                            precise=precise, meta=meta)
@@ -316,22 +334,23 @@ _EDGE_LENS = [1, 3, 4, 5, 7, 8, 9, 12, 13, 15, 16, 17, 31, 32, 33, 47, 49, 55, 5
 
 
 @pytest.mark.parametrize("raw", [False, True], ids=["given", "raw"])
-@pytest.mark.parametrize("cus,chunk64", [(None, True), (4, True), (4, False)], ids=["whole", "lists", "chunk32"])
-def test_row_group_edges(oracle, raw, cus, chunk64):
-    """Sequences that end at, before and after every row-group edge, through each chunk kernel form with given and
-    in-kernel gates.  Bars as in the other parity tests: outputs 2e-2 x RMS beyond bf16 storage, states 1e-3."""
+@pytest.mark.parametrize("form", ["split", "whole", "lists", "chunk32"])
+def test_row_group_edges(oracle, raw, form):
+    """Sequences that end at, before and after every row-group edge, through each chunk kernel form (_form_meta) with
+    given and in-kernel gates.  Bars as in the other parity tests: outputs 2e-2 x RMS beyond bf16 storage, states
+    1e-3."""
     if not raw:
-        _plain_case(oracle, 2, _EDGE_LENS, 140, cus=cus, chunk64=chunk64)
+        _plain_case(oracle, 2, _EDGE_LENS, 140, form=form)
         return
     kda = _kda()
     H, lens = 2, _EDGE_LENS
-    _say(f"row group edges, gates in the kernel, cus={cus} chunk64={chunk64}")
+    _say(f"row group edges, gates in the kernel, {form}")
     g = gen(141)
     q, k, v, raw_g, raw_b, A_log, dt_bias = _raw_inputs(g, sum(lens), H)
     h0 = torch.randn(len(lens), H, D, D, generator=g) * 0.05
-    meta = _list_meta(kda, lens, H, cus, chunk64) if cus else None
     o, fin = kda.kda_prefill(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), raw_g[None].to(DEV), raw_b[None].to(DEV),
-                             A_log.to(DEV), dt_bias.to(DEV), h0.to(DEV), torch.tensor(_cu(lens)).to(DEV), meta=meta)
+                             A_log.to(DEV), dt_bias.to(DEV), h0.to(DEV), torch.tensor(_cu(lens)).to(DEV),
+                             meta=_form_meta(kda, lens, H, form))
     torch.cuda.synchronize()
     qn, kn, vf, gl, bt = _oracle_gated(oracle, q, k, v, raw_g, raw_b, A_log, dt_bias)
     # the kernels raise log-decays below -9 to -9, which a one-token sequence's state shows (see the header)
@@ -341,14 +360,17 @@ def test_row_group_edges(oracle, raw, cus, chunk64):
         assert rel_frob(f32(fin[n]), rf[n]) <= STATE_TOL, f"seq {n} (len {lens[n]})"
 
 
-@pytest.mark.parametrize("form", ["whole", "precise", "lists", "chunk32"])
-def test_correlated_keys(oracle, form):
+@pytest.mark.parametrize("form,precise", [("split", False), ("whole", False), ("lists", False), ("chunk32", False),
+                                          ("split", True), ("whole", True)])
+def test_correlated_keys(oracle, form, precise):
     """Keys with a common direction (cosines ~0.5), beta ~0.9 and hardly any decay: the 16 x 16 systems I + L of the
     solve are far from the identity (entries ~0.45 everywhere below the diagonal), so every block and row of their
-    inverses counts; lengths end inside and at the edges of the 4-row blocks.  Bars as in the other parity tests."""
+    inverses counts; lengths end inside and at the edges of the 4-row blocks.  Through each chunk kernel form
+    (_form_meta).  Bars as in the other parity tests; they hold without the precise mode's low parts too, so that what
+    the mode adds is not seen here."""
     kda = _kda()
     H, lens = 2, [1, 4, 5, 15, 16, 17, 31, 33, 50, 64, 77, 200]
-    _say(f"correlated keys, {form}")
+    _say(f"correlated keys, {form}" + (" precise" if precise else ""))
     g = gen(142)
     T = sum(lens)
     q = torch.randn(T, H, D, generator=g).bfloat16()
@@ -357,11 +379,9 @@ def test_correlated_keys(oracle, form):
     gl = -1e-3 * torch.rand(T, H, D, generator=g)
     bt = 0.85 + 0.1 * torch.rand(T, H, generator=g)
     h0 = torch.randn(len(lens), H, D, D, generator=g) * 0.05
-    cus = None if form in ("whole", "precise") else 4
-    meta = _list_meta(kda, lens, H, cus, form != "chunk32") if cus else None
     o, fin = kda.chunk_kda(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), gl[None].to(DEV), bt[None].to(DEV),
                            initial_state=h0.to(DEV), output_final_state=True, cu_seqlens=torch.tensor(_cu(lens)).to(DEV),
-                           precise=form == "precise", meta=meta)
+                           precise=precise, meta=_form_meta(kda, lens, H, form))
     torch.cuda.synchronize()
     ro, rf = oracle.prefill_plain(f32(q), f32(k), f32(v), f32(gl), f32(bt), _cu(lens), initial_state=f32(h0), precision=64)
     _check_out(o[0], ro, "correlated keys", _cu(lens))
