@@ -155,6 +155,12 @@ __device__ __forceinline__ void split_bf16x2(float x0, float x1, uint32_t& hi, u
     const bf16x2_t m10 = __builtin_bit_cast(bf16x2_t, c10), m01 = __builtin_bit_cast(bf16x2_t, c01);
     lo = f2bf2(__builtin_amdgcn_fdot2_f32_bf16(hp, m10, x0, false), __builtin_amdgcn_fdot2_f32_bf16(hp, m01, x1, false));
 }
+// Before an fp16 hi + lo split of x: keeps x in a register, so that hi = RNE(x) and the hi inside lo = RNE(x - hi) are one
+// value.  Without it the compiler may form one of the two straight from the multiplication that made x
+// (v_fma_mixlo_f16, one rounding) and the other from the product rounded to fp32: where that lands on a tie of fp16 they
+// differ by an ulp of hi, which the pair is then off by (2 of 73 k right-hand side values of a test; the state of their
+// head 1.4e-5 off instead of 2.7e-7).
+__device__ __forceinline__ void one_rounding(float& x) { asm("" : "+v"(x)); }
 __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t (&w)[4]) {
     return __builtin_bit_cast(bf16x8, u32x4{w[0], w[1], w[2], w[3]});
 }
@@ -832,13 +838,15 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     aq[e] = (half_t)((4 * g + e <= m) ? aqk[e] : 0.f);
                 *reinterpret_cast<f16x4*>(&sAq[half_at(i, pos64(16 * I + 4 * g), RST, AQ_HALF)]) = aq;
                 // T_II = (I + L_II)^-1 of this wave's block while waves 4..7 still work on the off-diagonal blocks
-                const f32x4 x = invert_unit_lower(sL + I * 16 * 20, g, m);
+                const f32x4 x4 = invert_unit_lower(sL + I * 16 * 20, g, m);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const half_t hi = (half_t)x[e];
+                    float x = x4[e];
+                    if (PREC) one_rounding(x);
+                    const half_t hi = (half_t)x;
                     sAk[(16 * I + 4 * g + e) * RS16S + 16 * I + m] = hi;
                     // PREC: the low part over the gate totals, which nothing reads until the next chunk's
-                    if (PREC) sTl[(16 * I + 4 * g + e) * 16 + m] = (half_t)(x[e] - (float)hi);
+                    if (PREC) sTl[(16 * I + 4 * g + e) * 16 + m] = (half_t)(x - (float)hi);
                 }
             } else {
                 // block row I, NJ column blocks from J0 (compile-time: one straight-line copy per wave)
@@ -886,7 +894,8 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                         f16x4 ak, al, aq;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const float x = nb * akk[t][e];
+                            float x = nb * akk[t][e];
+                            if (PREC) one_rounding(x);
                             ak[e] = (half_t)x;
                             al[e] = (half_t)(x - (float)ak[e]);
                             aq[e] = (half_t)aqk[t][e];
@@ -957,7 +966,12 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 f16x4 Xh[4], Xl[4], Uh[4], Ul[4];
                 auto split4 = [](const f32x4& x, f16x4& hi, f16x4& lo) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) { hi[e] = (half_t)x[e]; lo[e] = (half_t)(x[e] - (float)hi[e]); }
+                    for (int e = 0; e < 4; ++e) {
+                        float y = x[e];
+                        if (PREC) one_rounding(y);
+                        hi[e] = (half_t)y;
+                        lo[e] = (half_t)(y - (float)hi[e]);
+                    }
                 };
 #pragma unroll
                 for (int I = 0; I < 4; ++I) {

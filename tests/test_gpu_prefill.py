@@ -389,6 +389,45 @@ def test_correlated_keys(oracle, form, precise):
         assert rel_frob(f32(fin[n]), rf[n]) <= STATE_TOL, f"seq {n} (len {lens[n]})"
 
 
+@pytest.mark.parametrize("form", ["whole", "split"])
+def test_precise_low_parts(oracle, form):
+    """What precise=True adds, on sequences of one chunk where its fp16 pairs are all that rounds: no start state (the
+    fp16 W and S do not enter), no decay, and keys of 64 channels +-1/8 with a common direction (cosines ~0.64), so that
+    the normalized keys, the gated operands and Kd^T are exact.  The state error is then 1e-7 (fp32 sums and pairs of 22
+    bits).  Emulated roundings give 1.3e-4 or more on the sequences over 16 tokens when any one of the pairs (-A_IJ,
+    T_II, the right-hand side, X_J, V') loses its low part, 4e-4 when all do; two values whose low
+    part belonged to another rounding of the high part showed as 1e-5.  The bar is 5e-6, and the default mode must miss
+    it.  split: beside a long sequence cut into pieces, so that the kernel with transitions walks them."""
+    kda = _kda()
+    H, lens = 2, [1, 4, 5, 15, 16, 17, 31, 33, 49, 50, 64]
+    short, end = len(lens), sum(lens)
+    if form == "split":
+        lens = lens + [512]
+    _say(f"precise low parts, {form}")
+    g = gen(143)
+    T = sum(lens)
+    base = torch.sign(torch.randn(1, H, D, generator=g))
+    base[..., ::2] = 0
+    k = (base * torch.where(torch.rand(T, H, D, generator=g) < 0.1, -1.0, 1.0) * 0.125).bfloat16()
+    q, v = torch.randn(T, H, D, generator=g).bfloat16(), torch.randn(T, H, D, generator=g).bfloat16()
+    gl = torch.zeros(T, H, D)
+    bt = 0.85 + 0.1 * torch.rand(T, H, generator=g)
+    ro, rf = oracle.prefill_plain(f32(q), f32(k), f32(v), f32(gl), f32(bt), _cu(lens), precision=64)
+    meta = _form_meta(kda, lens, H, form)
+    err = {}
+    for precise in (True, False):
+        o, fin = kda.chunk_kda(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), gl[None].to(DEV), bt[None].to(DEV),
+                               output_final_state=True, cu_seqlens=torch.tensor(_cu(lens)).to(DEV), precise=precise,
+                               meta=meta)
+        torch.cuda.synchronize()
+        _check_out(o[0][:end], ro[:end], f"precise low parts, precise={precise}", _cu(lens[:short]))
+        err[precise] = [rel_frob(f32(fin[n]), rf[n]) for n in range(short)]
+        _say(f"precise={precise}: " + " ".join(f"{e:.1e}" for e in err[precise]))
+    for n in range(short):
+        assert err[True][n] <= 5e-6, f"seq {n} (len {lens[n]}): {err[True][n]:.3e}"
+        assert err[False][n] <= STATE_TOL and (lens[n] <= 16 or err[False][n] > 5e-6), f"seq {n}: {err[False][n]:.3e}"
+
+
 def _pages(slots, H, taps, g):
     """vLLM hybrid page layout (kda/mi350x/CONTRACT.md:60-67): conv state then SSM state per padded page."""
     dim = H * D
