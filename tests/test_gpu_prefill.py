@@ -100,11 +100,12 @@ def test_varlen_with_initial_states(oracle):
 
 
 def test_precise_mode_whole_and_split(oracle):
-    """precise=True (fp16-pair operands in the solve and the state updates) on whole sequences and on a layout cut
+    """precise=True (fp16-pair operands in the solve and the state updates) on whole sequences and on layouts cut
     into pieces (later pieces carry their transition, whose update takes the pair too), and on a plan that chose the
     32-token kernel (which has no precise form: the launch runs the 64-token kernel on the plan's workgroup lists),
     against the fp64 oracle."""
-    _plain_case(oracle, 4, [300, 64, 1, 1000, 77], 1, precise=True)
+    _plain_case(oracle, 4, [300, 64, 1, 1000, 77], 1, precise=True, form="whole")
+    _plain_case(oracle, 4, [300, 64, 1, 1000, 77], 1, precise=True, form="split")
     _plain_case(oracle, 2, [8192, 300], 70, precise=True)
     _plain_case(oracle, 2, [600, 300, 130, 1, 0, 65, 700, 33], 71, precise=True, cus=4, chunk64=False)
 
@@ -438,18 +439,19 @@ def _pages(slots, H, taps, g):
     return raw, ssm
 
 
-@pytest.mark.parametrize("cus,chunk64", [(None, True), (4, True), (4, False)], ids=["whole", "lists", "chunk32"])
-def test_serving_pool_checkpoints_page_layout(oracle, cus, chunk64):
+@pytest.mark.parametrize("form", ["split", "whole", "lists", "chunk32"])
+def test_serving_pool_checkpoints_page_layout(oracle, form):
     """prefill_prepare + prefill on the page layout: has_initial_state with NaN rows, one checkpoint per sequence,
-    strided raw_beta, out a slice behind 256 leading rows; only out and the named rows change.  cus = 4: 28 items for
-    4 CUs, run as the 64-token kernel's workgroup lists (7 items per list, gates in the kernel: each item's dt_bias
-    handed to the next) and as the 32-token kernel (one workgroup per item)."""
+    strided raw_beta, out a slice behind 256 leading rows; only out and the named rows change.  split: the plan
+    prefill_prepare makes.  lists, chunk32: 28 items for 4 CUs, run as the 64-token kernel's workgroup lists (7 items per
+    list, gates in the kernel: each item's dt_bias handed to the next) and as the 32-token kernel (one workgroup per
+    item)."""
     kda = _kda()
     H = 4
     lens = [777, 64, 1, 130, 1024, 17, 255]
     hinit = [1, 0, 1, 0, 1, 1, 0]
     ck_off = [704, 64, 0, 0, 1024, 0, 192]
-    _say(f"serving pool H={H} lens={lens} cus={cus} chunk64={chunk64}")
+    _say(f"serving pool H={H} lens={lens} {form}")
     g = gen(40)
     T, N = sum(lens), len(lens)
     q, k, v, raw_g, raw_b, A_log, dt_bias = _raw_inputs(g, T, H)
@@ -473,8 +475,11 @@ def test_serving_pool_checkpoints_page_layout(oracle, cus, chunk64):
     out = parent[:, 256:256 + T]
     parent_before = parent.clone()
     cu_cpu = torch.tensor(_cu(lens), dtype=torch.int32)
-    meta = (kda.prefill_prepare(cu_cpu, H, torch.tensor(ck_off, dtype=torch.int32), cidx, device=DEV) if cus is None
-            else _list_meta(kda, lens, H, cus, chunk64, checkpoint_offsets=torch.tensor(ck_off, dtype=torch.int32)))
+    if form == "split":
+        meta = kda.prefill_prepare(cu_cpu, H, torch.tensor(ck_off, dtype=torch.int32), cidx, device=DEV)
+        assert meta.split != (0, 0), meta.split
+    else:
+        meta = _form_meta(kda, lens, H, form, checkpoint_offsets=torch.tensor(ck_off, dtype=torch.int32))
     kda.prefill(q[None].to(DEV), k[None].to(DEV), v[None].to(DEV), raw_g[None].to(DEV), beta_view, A_log.to(DEV),
                 dt_bias.to(DEV), D ** -0.5, -5.0, ssm, sidx.to(DEV), torch.tensor(hinit, dtype=torch.bool).to(DEV),
                 cu_cpu.to(DEV), out, torch.tensor(ck_off, dtype=torch.int32).to(DEV), cidx.to(DEV), meta=meta)
