@@ -2,7 +2,7 @@
 //
 // chunk_kernel keeps a 64-token chunk's operands in 158 KiB of LDS, so a CU holds one workgroup: its 8 waves (two
 // per SIMD) meet at the same four barriers per chunk and stall together.  Here a chunk is 32 tokens, the row arrays
-// halve and the workgroup needs 72 KiB, so two independent workgroups share a CU: still two waves per SIMD, but from
+// halve and the workgroup needs 75.2 KiB, so two independent workgroups share a CU: still two waves per SIMD, but from
 // workgroups whose barriers and dependent chains do not line up.  Per token the work is the same (the Gram and solve
 // blocks shrink with the chunk; the per-chunk state work -- decay, fp16 copies of S -- doubles).  Each wave keeps a
 // 128 x 32 slice of S (64 VGPRs), so a piece that also carries its transition does not fit: this kernel runs unsplit

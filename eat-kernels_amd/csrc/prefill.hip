@@ -167,7 +167,7 @@ __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t (&w)[4]) {
 // 2^x (v_exp_f32)
 __device__ __forceinline__ float exp2_(float x) { return __builtin_amdgcn_exp2f(x); }
 // sigmoid through the hardware reciprocal (v_rcp_f32, within 1 ulp): the IEEE division of sigmoidf_ is a sequence of
-// about ten instructions, and the raw-row phase takes 17 sigmoids per thread and chunk
+// about ten instructions, and the front takes 17 sigmoids per thread and chunk
 __device__ __forceinline__ float sigmoid_rcp(float x) { return __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
 // A per-token log-decay below KDA355_MIN_LOG_DECAY (-9) is raised to it: the diagonal Gram blocks hold e^{+-8 g} over
 // 8 tokens, inside 2^{+-104} for g >= -9, where the factors and the low halves of their bf16 pairs stay normal (the
@@ -534,8 +534,9 @@ struct ItemWords {
 // lo = RNE(x - hi): 22 bits) instead of single fp16 values: -A_IJ, T_II, the solved blocks X_J, the right-hand side
 // before T_II, and V' (-W P for a transition).  On chunks of nearly parallel keys with beta ~ 1 the substitution
 // cancels, and these single roundings set the state error: the reference eval's deep-layer probe measures 9.3e-4
-// relative Frobenius with single operands and 4.9e-4 with the pairs; config 1 takes ~11 % longer (more MFMAs in the
-// dependent chain of the solve, twice as many in the state update).
+// relative Frobenius with single operands and 4.9e-4 with the pairs.  8 x 4904 tokens, H 32, takes 735 us instead of
+// 628, 131,072 tokens 3079 instead of 2679 (more MFMAs in the dependent chain of the solve, 2.1 k -> 4.5 k cycles a chunk;
+// twice as many in the state update, walk 4.1 k -> 4.9 k).
 template <bool RG, bool P1, bool PREC>
 __global__ void __launch_bounds__(PF_THREADS, 1)
     chunk_kernel(PfParams p, const int32_t* __restrict__ tab, const int32_t* __restrict__ ck_idx, int list_off) {
@@ -550,7 +551,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     half_t* sAq = reinterpret_cast<half_t*>(lds + LDS_AQ);   // A_qk (columns permuted)
     half_t* sAk = reinterpret_cast<half_t*>(lds + LDS_AK);   // -A_kk off-diagonal blocks, T_II diagonal blocks
     float* sL = reinterpret_cast<float*>(lds + LDS_L);       // -L_II diagonal blocks, column-major [4][16][20]
-    float* sF = reinterpret_cast<float*>(lds + LDS_F);       // per-channel factors [18][128]
+    float* sF = reinterpret_cast<float*>(lds + LDS_F);       // per-channel factors [18][RSF]
     float* sWt = reinterpret_cast<float*>(lds + LDS_WT);     // gate totals of the 8 waves' rows [8][128]
     half_t* sTl = reinterpret_cast<half_t*>(lds + LDS_WT);   // PREC: T_II's low parts [64][16], after the factors
     float* sBeta = reinterpret_cast<float*>(lds + LDS_BETA);
@@ -659,7 +660,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
     load_start_state(state_source(cur));
 
     const int ck_mode = (p.flags & KDA355_PF_CK_EVERY) ? 2 : ((p.flags & KDA355_PF_CK_SINGLE) ? 1 : 0);
-    // gate-in-kernel constants for this thread's 16 channels
+    // gate-in-kernel constants: An of the head, An dt_bias of the channel tid
     float An = 0.f;
     if (RG) {
         An = gate_an(cur.alog);
@@ -916,10 +917,10 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                 else
                     off_diagonal(integral_constant<int, 3>{}, integral_constant<int, 2>{}, integral_constant<int, 1>{});
             }
-            // The initial state loads (issued in the prologue or at the item's start) complete here, before any
-            // next-chunk row is in flight: an empty use of S makes the compiler's wait for them fall at this point,
-            // where in every later chunk only the long-finished output stores are outstanding, instead of before each
-            // walk, where it would also wait for the prefetched rows.
+            // The initial state loads (issued in the prologue or at the item's start) complete here: an empty use of S
+            // makes the compiler's wait for them fall at this point.  It waits by count for everything older than the
+            // next chunk's 8 q and k loads, which stay in flight; in later chunks that is the long-finished output
+            // stores.  Before the walk it would also wait for the rows loaded since.
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) asm volatile("" : "+v"(S[dt]));
             load_rows_vb(p, pf_h, pf_t, pf_L, row0, c4, RB, nx);
@@ -1024,7 +1025,7 @@ __global__ void __launch_bounds__(PF_THREADS, 1)
                     }
                 }
             }
-            // the next item's gate dt_bias for its first raw-row phase (this chunk's has read sDT; the barrier below
+            // the next item's gate dt_bias for its first chunk's front (this chunk's has read sDT; the barrier below
             // publishes the new values)
             if (RG && !pf_here && more && tid < D) sDT[tid] = dtb_next;
             lds_barrier();
