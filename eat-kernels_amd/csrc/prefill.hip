@@ -1725,15 +1725,20 @@ extern "C" int kda355_prefill_plan(const KdaPrefillPlanIn* in, KdaPrefillPlan* p
     // ceil(nch / T) near-equal pieces, or into pieces of T chunks followed by the remainder (which fills CUs the long
     // pieces leave idle: 16 chunks on 3/4 of the CUs cut as 12 + 4), for T on a geometric ladder from a quarter of the
     // balanced per-CU load.  Pieces have >= MIN_PIECE chunks in a first pass and >= 1 in a second, whose candidates
-    // must beat the first pass's best.  Each candidate is costed in chunk times (one chunk of one head on one CU,
-    // ~11 us) by list-scheduling its workgroups in launch order onto the CUs of the shader engine each one is sent to
-    // (later pieces cost as much per chunk as first ones), plus the passes a split adds: the scan, sequential over the
-    // pieces of a sequence (SCAN_BASE + STEP_UNITS per later piece of the most-cut sequence, + SCAN_WG_UNITS per scan
-    // workgroup per CU: 8 per split sequence and head), and the output fixup (FIX_BASE + FIX_UNITS per chunk-head of
-    // later pieces, spread over the chip); every workgroup also pays a start-up of START_QUARTERS / 4 chunk times.  The cheapest candidate wins; ties keep fewer pieces.  The
-    // first piece of a split sequence runs from the true start state; later pieces run from S = 0, carry their
-    // transition and are completed by the scan, fixup and checkpoint-compose kernels.  Measured on MI355X: the scan
-    // ~7 us to start and ~0.55 us a step, the fixup ~11 ns per chunk-head.
+    // must beat the first pass's best.  Each candidate is costed in chunk times (one chunk of one head on one CU, in later
+    // pieces as much as in first ones) by list-scheduling its workgroups in launch order onto the CUs of the shader engine
+    // each one is sent to, plus the passes a split adds: the scan, sequential over the pieces of a sequence (SCAN_BASE +
+    // STEP_UNITS per later piece of the most-cut sequence, + SCAN_WG_UNITS per scan workgroup per CU: 8 per split sequence
+    // and head), and the output fixup (FIX_BASE + FIX_UNITS per chunk-head of later pieces, spread over the chip); every
+    // workgroup also pays a start-up of START_QUARTERS / 4 chunk times.  The cheapest candidate wins; ties keep fewer
+    // pieces.  The first piece of a split sequence runs from the true start state; later pieces run from S = 0, carry
+    // their transition and are completed by the scan, fixup and checkpoint-compose kernels.
+    // The constants were fitted to an older form of the chunk kernel, whose chunk took ~11 us.  Measured on MI355X with the
+    // present one: a chunk 7.0 us without and 7.4-7.9 us with a transition; start-up and end of a workgroup 12 us; the scan
+    // 5.2 us for 4 pieces, 14 for 16, 26 for 32 (H 4), 11-13 us for 8 pieces at H 32 (costed as 1.2 chunk times = 8.4 us);
+    // the fixup 4 us at least and 8.6-9.6 ns per chunk-head (costed as 3.5 us and 8.4 ns).  So all but the fixup are costed
+    // too low by a quarter to a half.  The choice has not suffered on the layouts tried: of 18-75 forced cuts of each of
+    // seven split layouts (1 to 12 sequences, 1024 to 131,072 tokens, H 4 to 96) none ran faster than the plan's.
     constexpr int MIN_PIECE = 2;  // the shortest piece of the first pass (the second allows one chunk)
     constexpr double SCAN_BASE = 0.6, STEP_UNITS = 0.05, SCAN_WG_UNITS = 0.25, FIX_BASE = 0.5, FIX_UNITS = 0.0012;
     constexpr int64_t START_QUARTERS = 4;  // a workgroup's start-up (state, first rows): about one chunk time
@@ -1932,10 +1937,11 @@ extern "C" int kda355_prefill_plan(const KdaPrefillPlanIn* in, KdaPrefillPlan* p
         // first 2 x num_cus dealt two to a CU and every later one to the CU that frees a slot first.  A workgroup
         // advances C32_PAIRED chunk times per 64 tokens while it shares its CU and C32_ALONE when alone, plus
         // C32_START of start-up, in chunk times of the 64-token kernel.  The constants are a least-squares fit (in
-        // log ratio) to eleven layouts timed on MI355X with both kernels: 384-1024 items of 2-32 chunks, where the
-        // 32-token kernel runs 3-11 % faster, a ragged layout 8 % slower, the 5-47-chunk p96 layouts 28-35 % slower
-        // (long chains alone on their CUs).  It is used when this simulated span beats the 64-token kernel's best
-        // (lists or one workgroup per item) by 3 %.
+        // log ratio) to eleven layouts timed on MI355X with older forms of both kernels: 384-1024 items of 2-32 chunks,
+        // where the 32-token kernel ran 3-11 % faster, a ragged layout 8 % slower, the 5-47-chunk layouts of 96 heads
+        // 28-35 % slower (long chains alone on their CUs).  With the present forms six of those layouts read 3-10 % faster
+        // and the ragged one 1 % slower, so the choices stand.  It is used when this simulated span beats the 64-token
+        // kernel's best (lists or one workgroup per item) by 3 %.
         constexpr double C32_ALONE = 1.2, C32_PAIRED = 1.85, C32_START = 0.3;
         struct Cu { double t = 0, w[2] = {0, 0}; int n = 0, ver = 0; };
         std::vector<Cu> cu(num_cus);
