@@ -184,7 +184,7 @@ int kda355_decode_launch(const KdaDecodeArgs* args, kda355_stream_t stream);
                                       before token j * ck_every, stored to ck_pool[ck_idx[row_start_n + j]] with
                                       row_start_n = sum of the earlier sequences' row counts (kda/b200/kda_b200.py:19-22) */
 #define KDA355_PF_PRECISE 64u      /* the solve's and the state update's fp16 operands as fp16 pairs (22 bits): about half
-                                      the state error on chunks of nearly parallel keys with beta ~ 1, ~11 % more time.
+                                      the state error on chunks of nearly parallel keys with beta ~ 1, 3-17 % more time.
                                       No counterpart in the reference (its prefill precision is fixed). */
 #define KDA355_PF_CHUNK64 128u     /* keep the 64-token kernel (and the plan's workgroup lists) where the plan chose the
                                       32-token kernel (KdaPrefillPlan.chunk32); a comparison and test switch.  No
